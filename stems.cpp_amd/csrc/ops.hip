@@ -763,6 +763,8 @@ __global__ __launch_bounds__(256) void ew_flat_kernel(const float* __restrict__ 
 // Paths, by shape:
 //   single pass (gn_fused_kernel) when the groups fit on the device at once, VEC < 4 and y
 //     does not overlap x: x is read once, the blocks exchange their partial sums (grid_sync.hpp);
+//   one block per group (gn_group_kernel) for more than kGridMaxGroups groups of at most 65,536
+//     floats;
 //   two passes otherwise: gn_partial_kernel writes each chunk's partial sums (and K), then
 //     gn_apply_kernel folds its group's partials itself (or reads gn_fold_kernel's totals when
 //     a group has more than kGnFoldDirect chunks) and writes its chunk.
@@ -1204,6 +1206,133 @@ __global__ __launch_bounds__(kGnThreads) void gn_apply_kernel(GroupNormArgs a) {
     else gn_apply_body<AK, GELU, VEC, false>(a, gt, begin, count, c0, i3, lo, red);
 }
 
+// One block per group, for launches of many small groups (the frequency branch's rows: 512 groups of
+// 2,016 or 32,256 floats): the group stays in registers between its sums and its output, so x is
+// read once, in one launch, and the blocks exchange nothing. Half h of the block (512 threads)
+// holds float4 t of chunks h, h + H, ... of gn_chunk<1>() floats, H = NT / 512; a chunk's wave sums,
+// the waves of a chunk in order and lane_sum over the chunks are the sums of the other paths in
+// their order (block_sum2_n of one wave's values and seven +0.0), so the bits are theirs. Bound by
+// the read and the write of x: [336, 96, 512] 28.3 us, 4.7 TB/s, the rate of a plain copy (two passes with per-element
+// parameters 99 + 20 us); [336, 6, 512] with GELU 6.7 us (12.4 + 4.2). The affine parameters (per channel) are staged in LDS, two channels a float4 at most (planes of 4 floats up).
+// 512 threads x 16 float4 (64 values in registers) leave two blocks a CU; groups of 32,769 to
+// 65,536 floats take 1,024 threads, larger ones the two passes. y may be x: a thread writes the
+// elements it read.
+constexpr int kGnGroupMaxChannels = 1024;
+constexpr int kGnGroupMaxChunks = 32;
+
+template <bool AFF, bool GELU, int NT, int K, bool VECT>
+__device__ __forceinline__ void gn_group_body(const GroupNormArgs& a, const float* xg, float* yg, unsigned count,
+                                              const float* wl, const float* bl, unsigned nc, double (*red)[8][2]) {
+    constexpr int H = NT / kGnThreads;
+    const unsigned half = threadIdx.x / kGnThreads, t = threadIdx.x % kGnThreads;
+    float v[K][4];
+    const double shift = (double)xg[0];
+    // 32-bit byte offsets from the group's base (a group has at most 2^18 bytes).
+    const char* xb = reinterpret_cast<const char*>(xg);
+#pragma unroll
+    for (int m = 0; m < K; m++) {
+        const unsigned p = (m * H + half) * gn_chunk<1>() + t * 4;
+        if constexpr (VECT) {
+            const float4 q = *reinterpret_cast<const float4*>(xb + 4 * min(p, count - 4));
+            v[m][0] = q.x;
+            v[m][1] = q.y;
+            v[m][2] = q.z;
+            v[m][3] = q.w;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[m][j] = *reinterpret_cast<const float*>(xb + 4 * min(p + j, count - 1));
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < K; m++) {
+        const unsigned c = m * H + half, p = c * gn_chunk<1>() + t * 4;
+        double s1 = 0.0, s2 = 0.0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const double d = p + j < count ? (double)v[m][j] - shift : 0.0;
+            s1 = s1 + d;
+            s2 = fma(d, d, s2);
+        }
+        s1 = lane_sum<kWave>(s1);
+        s2 = lane_sum<kWave>(s2);
+        if (t % kWave == 0) {
+            red[c][t / kWave][0] = s1;
+            red[c][t / kWave][1] = s2;
+        }
+        __builtin_amdgcn_sched_barrier(0);                     // a chunk's doubles at a time
+    }
+    // Opaque: the values themselves stay in registers, not their conversions to double, and not
+    // the offsets and channels of all K float4.
+    unsigned p0 = half * gn_chunk<1>() + t * 4;
+#pragma unroll
+    for (int m = 0; m < K; m++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) asm volatile("" : "+v"(v[m][j]));
+    __syncthreads();                                           // also publishes wl and bl
+    // Every wave adds the chunks for itself: lane c the waves of chunk c, then the lanes.
+    const unsigned lane = threadIdx.x % kWave;
+    double t1 = 0.0, t2 = 0.0;
+    if (lane < (unsigned)(K * H)) {
+#pragma unroll
+        for (int w = 0; w < kGnThreads / kWave; w++) {
+            t1 += red[lane][w][0];
+            t2 += red[lane][w][1];
+        }
+    }
+    double mean, rstd;
+    gn_moments(lane_sum<kWave>(t1), lane_sum<kWave>(t2), count, shift, a.eps, mean, rstd);
+    char* yb = reinterpret_cast<char*>(yg);
+#pragma unroll
+    for (int m = 0; m < K; m++) {
+        asm volatile("" : "+v"(p0));
+        const unsigned p = m * H * gn_chunk<1>() + p0;
+        if (p >= count) continue;
+        float o[4];
+        unsigned c = 0, bnd = ~0u;
+        double a0 = rstd, d0 = fma(-mean, rstd, 0.0), a1 = a0, d1 = d0;
+        if constexpr (AFF) {
+            c = a.plane_div.div(p);
+            bnd = (c + 1) * a.plane;
+            const unsigned n = min(c + 1, nc - 1);
+            a0 = rstd * (double)wl[c];
+            d0 = fma(-mean, a0, (double)bl[c]);
+            a1 = rstd * (double)wl[n];
+            d1 = fma(-mean, a1, (double)bl[n]);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const bool nx = AFF && p + j >= bnd;
+            o[j] = gn_out<GELU>(fma((double)v[m][j], nx ? a1 : a0, nx ? d1 : d0));
+        }
+        if constexpr (VECT) {
+            store_stream(reinterpret_cast<float4*>(yb + 4 * p), make_float4(o[0], o[1], o[2], o[3]));
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (p + j < count) store_stream(reinterpret_cast<float*>(yb + 4 * (p + j)), o[j]);
+        }
+        __builtin_amdgcn_sched_barrier(0);                     // as in gn_write: the GELUs one float4 at a time
+    }
+}
+
+template <bool AFF, bool GELU, int NT, int K>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void gn_group_kernel(GroupNormArgs a) {
+    __shared__ double red[K * (NT / kGnThreads)][8][2];
+    __shared__ float wl[AFF ? kGnGroupMaxChannels : 1], bl[AFF ? kGnGroupMaxChannels : 1];
+    long long begin, c0, i3;
+    unsigned count;
+    group_span(a, (int)blockIdx.x, begin, count, c0, i3);
+    const unsigned nc = (unsigned)min(a.cpg, a.ne2 - c0);
+    if constexpr (AFF) {
+        for (unsigned i = threadIdx.x; i < nc; i += NT) {
+            wl[i] = a.w.p ? a.w.p[c0 + i] : 1.f;
+            bl[i] = a.b.p ? a.b.p[c0 + i] : 0.f;
+        }
+    }
+    if (a.vec) gn_group_body<AFF, GELU, NT, K, true>(a, a.x + begin, a.y + begin, count, wl, bl, nc, red);
+    else gn_group_body<AFF, GELU, NT, K, false>(a, a.x + begin, a.y + begin, count, wl, bl, nc, red);
+}
+
 // ----------------------------------------------------------------------------- ROPE
 // ggml_rope_ext without YaRN (ext_factor 0): theta_i = freq_scale * pos * base^(-2i/n_dims),
 // cos and sin scaled by attn_factor. Mode 0 rotates adjacent pairs (2i, 2i+1), mode 2 (NEOX)
@@ -1493,6 +1622,11 @@ Affine make_affine(const stx_tensor* t, const stx_tensor* x, const char* what) {
     return f;
 }
 
+// An affine operand with one value per ne1 index (or none).
+bool per_ne1(const stx_tensor* t, const stx_tensor* x) {
+    return !t || (t->ne[0] == 1 && t->ne[1] == x->ne[1] && t->ne[2] == 1 && t->ne[3] == 1 && (t->ne[1] == 1 || t->nb[1] == 4));
+}
+
 struct GnPlan {
     long long cpg, groups, groups_total, span;
     int vec, nch;
@@ -1542,6 +1676,34 @@ void launch_gn_vec(const GroupNormArgs& g, const GnPlan& p, const GridSync& sync
     launch_check("gn_apply_kernel");
 }
 
+// Launches gn_group_kernel where it applies: more groups than the single pass takes (few groups
+// are spread over more CUs by it), every group in one block's registers, affine per channel or none.
+template <bool GELU>
+bool launch_gn_groups(const GroupNormArgs& g, const GnPlan& p, int ak, bool disjoint, hipStream_t s) {
+    const bool aff = g.w.p || g.b.p;
+    if (p.groups_total <= kGridMaxGroups || p.nch > kGnGroupMaxChunks || p.vec != 1 || !(disjoint || g.x == g.y)) return false;
+    if (aff && ((ak != AFF_CHANNEL && ak != AFF_CHANNEL_WAVE) || g.cpg > kGnGroupMaxChannels || g.plane < 4)) return false;
+    auto go = [&](auto affine, auto threads, auto chunks) {
+        constexpr bool A = decltype(affine)::value;
+        constexpr int NT = decltype(threads)::value, K = decltype(chunks)::value;
+        hipLaunchKernelGGL((gn_group_kernel<A, GELU, NT, K>), dim3((unsigned)p.groups_total), dim3(NT), 0, s, g);
+    };
+    auto sized = [&](auto affine) {
+        using std::integral_constant;
+        constexpr integral_constant<int, 512> one{};
+        if (p.nch <= 1) go(affine, one, integral_constant<int, 1>{});
+        else if (p.nch <= 2) go(affine, one, integral_constant<int, 2>{});
+        else if (p.nch <= 4) go(affine, one, integral_constant<int, 4>{});
+        else if (p.nch <= 8) go(affine, one, integral_constant<int, 8>{});
+        else if (p.nch <= 16) go(affine, one, integral_constant<int, 16>{});
+        else go(affine, integral_constant<int, 1024>{}, integral_constant<int, 16>{});
+    };
+    if (aff) sized(std::true_type{});
+    else sized(std::false_type{});
+    launch_check("gn_group_kernel");
+    return true;
+}
+
 // Single pass when the groups fit (at most kGridMaxGroups of at most kGridMaxBlocks chunks,
 // all resident together) and y does not overlap x; otherwise two passes. Both give the same
 // bits.
@@ -1567,20 +1729,29 @@ void group_norm(const stx_tensor* a, const stx_tensor* dst, int n_groups, float 
     g.shift = reinterpret_cast<double*>(w + p.shift_off);
     g.tot = reinterpret_cast<double*>(w + p.tot_off);
     g.part = reinterpret_cast<double*>(w + p.part_off);
+    // One plane per group and parameters along ne1 (group_norm_rows over rows, src/htdemucs.cpp:120-127):
+    // the same memory and groups as [ne0, 1, ne1] per group with the parameters per channel, whose
+    // index is one division a float4 instead of six 64-bit remainders an element.
+    const bool along1 = p.cpg == 1 && (weight || bias) && per_ne1(weight, a) && per_ne1(bias, a);
+    const long long cpg = along1 ? ta.ne[1] : p.cpg;
+    if (along1) {
+        if (weight) g.w.kind = AFF_CHANNEL;
+        if (bias) g.b.kind = AFF_CHANNEL;
+    }
     g.ne0 = (unsigned)ta.ne[0];
-    g.ne1 = (unsigned)ta.ne[1];
-    g.ne2 = ta.ne[2];
-    g.plane = (unsigned)(ta.ne[0] * ta.ne[1]);
+    g.ne1 = along1 ? 1u : (unsigned)ta.ne[1];
+    g.ne2 = along1 ? ta.ne[1] : ta.ne[2];
+    g.plane = (unsigned)(ta.ne[0] * g.ne1);
     g.rplane = 1.0 / (double)g.plane;
     g.rne0 = 1.0 / (double)g.ne0;
     g.plane_div = FastDiv(g.plane);
-    g.cpg = p.cpg;
-    g.groups = (int)p.groups;
+    g.cpg = cpg;
+    g.groups = along1 ? 1 : (int)p.groups;
     g.nch = p.nch;
     g.eps = eps;
     // Every group span starts at (i3 * ne2 + g * cpg) * plane floats.
     g.vec = aligned16(ta.data) && aligned16(td.data) && (g.cpg * (long long)g.plane) % 4 == 0 &&
-                    (ta.ne[3] == 1 || (g.ne2 * (long long)g.plane) % 4 == 0)
+                    (p.groups_total == g.groups || (g.ne2 * (long long)g.plane) % 4 == 0)
                 ? 1
                 : 0;
     const size_t nbytes = (size_t)nelem(ta) * 4;
@@ -1590,6 +1761,7 @@ void group_norm(const stx_tensor* a, const stx_tensor* dst, int n_groups, float 
     };
     int ak = fits(AFF_CHANNEL) ? AFF_CHANNEL : fits(AFF_NE0) ? AFF_NE0 : AFF_GENERAL;
     if (ak == AFF_CHANNEL && g.plane >= 256) ak = AFF_CHANNEL_WAVE;
+    if (gelu ? launch_gn_groups<true>(g, p, ak, single, s) : launch_gn_groups<false>(g, p, ak, single, s)) return;
     switch (ak * 2 + (gelu ? 1 : 0)) {
         case AFF_CHANNEL_WAVE * 2 + 1: launch_group_norm<AFF_CHANNEL_WAVE, true>(g, p, sync, single, s); break;
         case AFF_CHANNEL_WAVE * 2: launch_group_norm<AFF_CHANNEL_WAVE, false>(g, p, sync, single, s); break;

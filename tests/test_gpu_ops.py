@@ -197,6 +197,39 @@ def test_group_norm_paths_same_bits(device, ops, shape, G, gelu, monkeypatch):
         assert forced > 0
 
 
+# (torch shape, groups, parameters along): one group per block up to 32 chunks of 2,048 floats, its limits
+# (32,768 | 32,769.. | 65,536 | 65,568 floats, 1,024 | 1,025 channels, planes of 4 | 3 floats), unaligned
+# spans, a ragged last group, a batch, and 8 groups (the grid-synchronised pass).
+GN_GROUP_CASES = [((512, 6, 336), 512, "ne1"), ((20, 96, 336), 20, "ne1"), ((9, 16, 2048), 9, "ne1"), ((9, 331, 99), 9, "ne1"),
+                  ((10, 128, 512), 10, "ne1"), ((10, 96, 683), 10, "ne1"), ((33, 5, 333), 33, "ne1"), ((9, 1024, 5), 9, "ne1"),
+                  ((9, 1025, 5), 9, "ne1"), ((16, 7, 4), 16, "ne1"), ((16, 7, 3), 16, "ne1"), ((11, 1, 1), 11, "ne1"),
+                  ((8, 96, 336), 8, "ne1"), ((2, 6, 48, 85), 6, "ne1"), ((64, 1, 700), 16, "ne2"), ((47, 1, 301), 10, "ne2"),
+                  ((3, 14, 2, 130), 4, "ne2"), ((12, 3, 1000), 12, "none")]
+
+
+@pytest.mark.parametrize("shape,G,along", GN_GROUP_CASES)
+@pytest.mark.parametrize("gelu", [False, True])
+def test_group_norm_many_groups_same_bits(device, ops, shape, G, along, gelu):
+    """Launches of many groups: parameters per ne1 or ne2 index, given as such (one block per group, or per-channel
+    parameters in the other paths), give the bits of the same parameters spread over whole planes (the general
+    per-element path, two passes), also in place; and the oracle's values."""
+    x = randn(device, shape, sum(shape) + G, 1.3, 0.7)
+    C = shape[-2] if along == "ne1" else shape[-3]
+    small = (C, 1) if along == "ne1" else (C, 1, 1)
+    plane = (C, shape[-1]) if along == "ne1" else (C,) + tuple(shape[-2:])
+    w, b = (None, None) if along == "none" else (randn(device, small, 70), randn(device, small, 71))
+    y = host(stx.group_norm(x, G, 1e-5, w, b, gelu=gelu))
+    assert rel_err(y, ops.group_norm(host(x), G, 1e-5, None if w is None else host(w), None if b is None else host(b), gelu=gelu)) <= TOL
+    xc = x.clone()
+    stx.group_norm(xc, G, 1e-5, w, b, gelu=gelu, out=xc)
+    assert np.array_equal(host(xc), y)
+    if w is not None:
+        full = host(stx.group_norm(x, G, 1e-5, w.expand(plane).contiguous(), b.expand(plane).contiguous(), gelu=gelu))
+        assert np.array_equal(full, y)
+        one = host(stx.group_norm(x, G, 1e-5, None, b, gelu=gelu))
+        assert np.array_equal(one, host(stx.group_norm(x, G, 1e-5, None, b.expand(plane).contiguous(), gelu=gelu)))
+
+
 def test_group_norm_errors(device):
     import torch
     x = randn(device, (4, 1, 100), 10)
