@@ -4,7 +4,7 @@
 // crossings, cutoff 0.95 of the lower Nyquist), tabulated once over |x| in [0, half] at 2^15 + 2
 // points and interpolated linearly; each output sample sums, in double and in input order, the
 // weighted input samples within `half` of its position. Two kernels. The default one,
-// resample_phase_kernel (below), weights each output by its exact phase; the per-tap one,
+// resample_phase_kernel (below), weights each output by its exact phase, on the matrix cores; the per-tap one,
 // resample_kernel, chosen by STX_RESAMPLE_EXACT=1, computes the table on the host with the
 // reference's formula (so it is bit-identical), keeps it on the device, and does every per-tap
 // operation as the reference's double operation in the reference's order, so its output is
@@ -19,6 +19,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <numeric>
+#include <type_traits>
 #include <vector>
 
 #include "common.hpp"
@@ -28,13 +29,15 @@ struct stx_resampler {
     int src = 0, dst = 0;
     double ratio = 1.0, half = 0.0;
     double* d_table = nullptr;       // [kTableN + 2]
-    // Phase table (see resample_phase_kernel): dst = up * g, src = down * g.
-    int up = 0, down = 0;
+    // Phase tables (see resample_phase_kernel): dst = up * g, src = down * g, U = m up, D = m down.
+    int U = 0, D = 0;
     int omin = 0;                    // offset of tap 0 from floor(c)
-    int npairs = 0, rs = 0;          // phase pairs (up + 1) / 2; doubles per pair row
-    int width = 0, pitch = 0, lds_bytes = 0;  // staged input tile of resample_phase_kernel
-    double* d_pair = nullptr;        // [npairs][rs]: the pair's two weight rows interleaved
-    int4* d_prange = nullptr;        // [npairs]: each row's first and last tap
+    int groups = 0, ks = 0;          // groups of 16 phases; products per group
+    int width = 0, pitch = 0;        // staged row of one period
+    long long lds_max = 0;           // LDS per workgroup of the device
+    double* d_weights = nullptr;     // [groups][ks][64]
+    int* d_goff = nullptr;           // [groups]
+    int2* d_range = nullptr;         // [U]
 };
 
 namespace stx {
@@ -93,158 +96,211 @@ __global__ __launch_bounds__(256) void resample_kernel(ResampleArgs a) {
         if (k < C) store_stream(a.out + (size_t)k * a.out_n + i, (float)acc[k]);
 }
 
-// The same sums over weights that depend only on the output's phase. With dst = up g and
-// src = down g, output i = q + M up sits at c = i down / up = fq + M down + p / up, where
-// fq = floor(q down / up) and p = q down mod up, so its taps j = fq + M down + omin + k and their
-// weights (the reference's table interpolation at |j - c|) are row p of a table of up rows
-// computed once on the host. Those weights differ from the reference's, which it computes per
-// output from c = i / ratio with ratio rounded to double, by the rounding of c (below 1e-9 for
-// three hours of 48 kHz audio), so the output is within a few float ulps of the reference's
-// (SNR above 160 dB) instead of bit-identical; the per-tap division, table lookup and
-// interpolation of resample_kernel are gone, leaving an fma per tap and a conversion per staged
-// sample read (shared by a pair of phases, below).
+// The same sums over weights that depend only on the output's phase, as products on the matrix
+// cores. With dst = up g and src = down g, and U = m up, D = m down for a whole m, output
+// i = q + M U sits at c = i down / up = fq + M D + p / up, where fq = floor(q down / up) and
+// p = q down mod up, so its taps j = fq + M D + omin + k and their weights (the reference's table
+// interpolation at |j - c|) are row p of a table of up rows computed once on the host. Those
+// weights differ from the reference's, which it computes per output from c = i / ratio with ratio
+// rounded to double, by the rounding of c (below 1e-9 for three hours of 48 kHz audio), so the
+// output is within a few float ulps of the reference's (SNR above 160 dB) instead of bit-identical.
 //
-// A workgroup takes one channel and the 64 output groups M = m0 + lane, m0 = 64 blockIdx.x: all
-// outputs in [m0 up, (m0 + 64) up). It stages in LDS, for each lane, the input its outputs read:
-// row l holds j = (m0 + l) down + omin + r for r < width = down + ntap + kPhaseOverread (zeros
-// outside the input, which add nothing; neighbouring rows overlap by ntap + kPhaseOverread). Rows
-// are `pitch` floats apart, width rounded up to odd, so the lanes of a read fall in different
-// banks. 48 -> 44.1 kHz stages 62 KB: two workgroups of 16 waves, the most waves a CU holds.
+// Sixteen neighbouring outputs q = 16 g .. 16 g + 15 of a period read one window of 4 ks samples
+// that starts at F = f(16 g) and holds all their taps, so for 16 periods M the outputs are
+//   Y[M][q] = sum over s < 4 ks of X[M D + F + s] W_g[s][q],
+// ks products v_mfma_f64_16x16x4_f64 (double operands and sums; W_g is zero outside a phase's own
+// taps). A workgroup takes R = 16 T periods of one channel and stages in LDS one row of `width`
+// samples per period (neighbouring rows overlap; rows are `pitch` floats apart, 2 mod 4, so that the
+// 32 lanes that read 16 rows at two neighbouring samples touch 32 banks: no conflicts measured). A wave
+// takes groups g and all T tiles of 16 periods: a weight operand (one double a lane, 512 contiguous
+// bytes from the cache, a step of four ahead) feeds T products, a sample operand is one LDS read and
+// one conversion.
 //
-// Each wave takes pairs of neighbouring phases q0 = 2 jp, q1 = q0 + 1 (jp = wave, wave + 16, ...).
-// Their windows, at r = fq0 + s and r = fq1 + k, overlap but for a tap or two at each end, so a
-// lane converts each staged sample it reads once and feeds both sums. The host interleaves the
-// pair's weight rows by s (w0(s), w1(s)): eight common taps are two 64-byte scalar loads from one
-// row and four paired LDS reads. Taps in only one window (the pair's ranges, lo0..hi0 and
-// lo1..hi1 in s) go through a guarded loop, so no tap is summed that its phase's window lacks;
-// each sum still takes its taps in order. The last 1-7 common taps load one whole chunk (at most
-// 7 samples and weight pairs past them, inside the row and the padded table) and sum only their
-// own under uniform branches. An odd last phase is paired with itself; its second sum is not
-// stored.
+// The double matrix rate (69 TFLOP/s measured) is a floor of 16 ceil(U / 16) / U more outputs and
+// 4 ks / taps more taps than the sum needs (1.09 and 1.30 for 48 -> 44.1 kHz, 180 s stereo: 48 us); it
+// takes 81 us there, staging, weights and stores sharing the vector memory pipe (47 us without the
+// products). One fma per tap on the vector units, which this took the place of, issued a conversion
+// for every two fmas and waited on LDS (115 us), left waves idle at ratios of few phases (2 : 1, 60 s
+// stereo: 943 -> 52 us), and its tile of 64 whole periods did not fit at 44.1 -> 8 kHz (350 -> 34 us).
+// Measured and dropped: ten waves (one a group) instead of eight at 44.1 -> 48 kHz, 70 against 61 us;
+// rows staged through registers, 96 us; four tiles a wave, 92 us; weights held in registers by
+// persistent workgroups with the next tile's rows on their way, 85 us (96 registers spill, and the
+// compiler waits for the rows before the first LDS read).
+//
+// A zero weight times an infinity or NaN is NaN, where the phase's own window may have no such tap;
+// finite samples never give a sum that is not finite (weights of at most 1, doubles). So where a sum
+// is not finite the wave sums its outputs again, each over its own taps alone, in tap order.
 struct PhaseArgs {
     const float* in;                 // [C][n]
     float* out;                      // [C][out_n]
-    const double* w;                 // [npairs][rs]: (w0(s), w1(s)) for s < rs / 2
-    const int4* range;               // [npairs]: lo0, hi0, lo1, hi1 in s
+    const double* w;                 // [groups][ks][64]: lane l holds tap 4 s + l / 16 of phase 16 g + l mod 16
+    const int* goff;                 // [groups]: F
+    const int2* range;               // [U]: first and last tap of each phase, counted from its group's F
     long long n, out_n;
-    int up, down, omin, npairs, rs;
-    int width, pitch;                // staged samples per lane row; floats between rows (odd)
-    FastDiv fup;                     // q down / up (below 2^20)
+    int U, D, omin, groups, ks;
+    int width, pitch;                // staged samples per period; floats between rows (2 mod 4)
 };
 
-constexpr int kPhaseTile = 64;                       // output groups per workgroup, one per lane
-constexpr int kPhaseWaves = 16;                      // waves per workgroup, each over every 16th phase pair
-constexpr int kPhaseStage = 4;                       // staged loads in flight per lane
+constexpr int kPhaseMaxWaves = 8;                    // a multiple of the CU's four SIMDs
 constexpr long long kPhaseMaxWeights = 1 << 18;      // up * ntap above this: per-tap kernel
-constexpr int kPhaseOverread = 8;                    // staged samples and table weights past the last used
+constexpr long long kPhaseMaxTable = 1 << 20;        // doubles of the groups' tables above this: per-tap kernel
+constexpr int kPhaseUnroll = 4;                      // ks is a multiple of it
 
-// The weight table and the pair ranges do not change while the kernel runs: read through the
-// constant address space, a wave-uniform load of them is a scalar load into SGPRs.
-typedef const __attribute__((address_space(4))) double* ConstDoubles;
+// The table does not change while the kernel runs: read through the constant address space, a
+// wave-uniform load of it is a scalar load.
 typedef const __attribute__((address_space(4))) int* ConstInts;
+typedef __attribute__((address_space(1))) unsigned* GlobalWords;
+typedef __attribute__((address_space(3))) unsigned* LocalWords;
+typedef double stx_v4d __attribute__((ext_vector_type(4)));
 
-// Taps s0..s1 of which only some lie in each window: each summed where its window has it.
-__device__ __forceinline__ void pair_edge(const float* xr, ConstDoubles wp, int4 rg, int s0, int s1, double& a0,
-                                          double& a1) {
-    for (int s = s0; s <= s1; s++) {
-        const double x = (double)xr[s];
-        if (s >= rg.x && s <= rg.y) a0 = fma(wp[2 * s], x, a0);
-        if (s >= rg.z && s <= rg.w) a1 = fma(wp[2 * s + 1], x, a1);
-    }
-}
-
-__global__ __launch_bounds__(kPhaseWaves * 64) void resample_phase_kernel(PhaseArgs a) {
-    extern __shared__ float xs[];
-    const int c = (int)blockIdx.y;
-    const long long m0 = (long long)blockIdx.x * kPhaseTile;
-    const float* in = a.in + (size_t)c * a.n;
-    const int lane = (int)threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    // Each wave stages whole rows: the row's first input index and its bounds are the same for
-    // the wave, so a sample costs an offset and, at the input's ends only, a bounds test.
-    for (int l = wave; l < kPhaseTile; l += kPhaseWaves) {
-        const long long jb = (m0 + l) * a.down + a.omin;        // input index of r = 0
+// Stages rows [0, R) of the tile that starts at period m0: row l holds input (m0 + l) D + omin + r for
+// r < width, zeros outside the input. Each wave takes whole rows. A row inside the input goes
+// straight to LDS (64 samples an instruction, all in flight together; the caller waits for them),
+// one at the input's ends through registers with a bounds test.
+template <int R>
+__device__ __forceinline__ void phase_stage(const PhaseArgs& a, const float* in, long long m0, float* xs, int wave, int waves,
+                                            int lane) {
+    for (int l = wave; l < R; l += waves) {
+        const long long jb = (m0 + l) * a.D + a.omin;           // input index of r = 0
         const float* src = in + jb;
         float* dst = xs + l * a.pitch;
-        const bool inside = jb >= 0 && jb + a.width <= a.n;
-        const int rlo = (int)max(-jb, 0LL), rhi = (int)min(a.n - jb, (long long)a.width);   // r in [rlo, rhi) is input
-        for (int r0 = 0; r0 < a.width; r0 += 64 * kPhaseStage) {
-            float v[kPhaseStage];
-#pragma unroll
-            for (int u = 0; u < kPhaseStage; u++) {
-                const int r = r0 + u * 64 + lane;
-                v[u] = r < a.width && (inside || (r >= rlo && r < rhi)) ? src[r] : 0.0f;
-            }
-#pragma unroll
-            for (int u = 0; u < kPhaseStage; u++) {
-                const int r = r0 + u * 64 + lane;
-                if (r < a.width) dst[r] = v[u];
+        if (jb >= 0 && jb + a.width <= a.n) {
+            for (int r0 = 0; r0 < a.width; r0 += 64)
+                if (r0 + lane < a.width)
+                    __builtin_amdgcn_global_load_lds((GlobalWords)(src + r0 + lane), (LocalWords)(dst + r0), 4, 0, 0);
+        } else {
+            for (int r = lane; r < a.width; r += 64) {
+                const long long j = jb + r;
+                dst[r] = j >= 0 && j < a.n ? in[j] : 0.0f;
             }
         }
     }
+}
+
+// Writes group g's sums of T tiles of 16 periods (lane l's sums v are those of period
+// l / 16 + 4 v of a tile, phase l mod 16); outp is output 0 of the first period, xg the group's
+// window in its row and `left` the outputs from outp to the end.
+template <int T>
+__device__ __forceinline__ void phase_store(const PhaseArgs& a, const stx_v4d (&acc)[T], float* outp, int left, const float* xg,
+                                            int g, int lane) {
+    const int lm = lane & 15, lk = lane >> 4, q = 16 * g + lm;
+    bool bad = false;
+#pragma unroll
+    for (int t = 0; t < T; t++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) bad |= !isfinite(acc[t][v]);
+    if (__ballot(bad) != 0) {
+        // In a branch of its own, so that the stores of the usual case wait for nothing.
+        if (q >= a.U) return;
+        const int2 rg = a.range[q];
+        const double* w = a.w + (size_t)g * a.ks * 64 + lm;
+        for (int row = lk; row < 16 * T && row * a.U + q < left; row += 4) {
+            const float* xw = xg + row * a.pitch;
+            double y = 0.0;
+            for (int k = rg.x; k <= rg.y; k++) y = fma(w[(k >> 2) * 64 + (k & 3) * 16], (double)xw[k], y);
+            outp[row * a.U + q] = (float)y;
+        }
+        return;
+    }
+    if (q >= a.U) return;
+#pragma unroll
+    for (int t = 0; t < T; t++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int i = (16 * t + 4 * v + lk) * a.U + q;
+            if (i < left) outp[i] = (float)acc[t][v];
+        }
+}
+
+// Bounds of 128 registers keep the sums in architectural registers: with a larger budget the
+// compiler moves them to accumulation registers and back around every loop step.
+template <int T>
+__global__ __launch_bounds__(kPhaseMaxWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void resample_phase_kernel(PhaseArgs a) {
+    extern __shared__ float xs[];
+    constexpr int R = 16 * T;
+    const int c = (int)blockIdx.y;
+    const long long m0 = (long long)blockIdx.x * R;
+    const int lane = (int)threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int waves = (int)blockDim.x >> 6;
+    phase_stage<R>(a, a.in + (size_t)c * a.n, m0, xs, wave, waves, lane);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");            // this wave's rows have landed
     __syncthreads();
-    float* outc = a.out + (size_t)c * a.out_n;
-    const long long i0 = (m0 + lane) * a.up;
-    for (int jp = wave; jp < a.npairs; jp += kPhaseWaves) {
-        const int q0 = 2 * jp;
-        const int fq0 = (int)a.fup.div((unsigned)q0 * (unsigned)a.down);
-        const ConstInts rgp = (ConstInts)a.range + 4 * jp;
-        const int4 rg = make_int4(rgp[0], rgp[1], rgp[2], rgp[3]);
-        const ConstDoubles wp = (ConstDoubles)(a.w + (size_t)jp * a.rs);
-        const float* xr = xs + lane * a.pitch + fq0;
-        const int lo_u = min(rg.x, rg.z), hi_u = max(rg.y, rg.w);
-        int lo_i = max(rg.x, rg.z), hi_i = min(rg.y, rg.w);
-        if (lo_i > hi_i) lo_i = hi_u + 1, hi_i = hi_u;            // no common taps: all on the edge path
-        double a0 = 0.0, a1 = 0.0;
-        pair_edge(xr, wp, rg, lo_u, lo_i - 1, a0, a1);
-        int s = lo_i;
-        for (; s + 7 <= hi_i; s += 8) {
-            const ConstDoubles wc = wp + 2 * s;                  // one base, constant offsets: two 64-byte loads
-            const float* xc = xr + s;
+    float* outp = a.out + (size_t)c * a.out_n + m0 * a.U;
+    const int left = (int)min(a.out_n - m0 * a.U, (long long)R * a.U);
+    for (int g = wave; g < a.groups; g += waves) {
+        const int F = ((ConstInts)a.goff)[g];
+        stx_v4d acc[T];
 #pragma unroll
-            for (int t = 0; t < 8; t++) {
-                const double x = (double)xc[t];
-                a0 = fma(wc[2 * t], x, a0);
-                a1 = fma(wc[2 * t + 1], x, a1);
-            }
+        for (int t = 0; t < T; t++) acc[t] = stx_v4d{0.0, 0.0, 0.0, 0.0};
+        const float* xr = xs + (lane & 15) * a.pitch + F + (lane >> 4);
+        const int tile = 16 * a.pitch;
+        const double* wl = a.w + (size_t)g * a.ks * 64 + lane;
+        double wn[kPhaseUnroll];
+#pragma unroll
+        for (int u = 0; u < kPhaseUnroll; u++) wn[u] = wl[64 * u];
+        for (int s = 0; s < a.ks; s += kPhaseUnroll) {
+            double wc[kPhaseUnroll];
+            // The next step's weights in flight through this one's products (the last step
+            // re-reads its own).
+            const double* wx = wl + 64 * (s + kPhaseUnroll < a.ks ? s + kPhaseUnroll : s);
+#pragma unroll
+            for (int u = 0; u < kPhaseUnroll; u++) wc[u] = wn[u];
+#pragma unroll
+            for (int u = 0; u < kPhaseUnroll; u++) wn[u] = wx[64 * u];
+            float x[kPhaseUnroll][T];
+#pragma unroll
+            for (int t = 0; t < T; t++)
+#pragma unroll
+                for (int u = 0; u < kPhaseUnroll; u++) x[u][t] = xr[t * tile + 4 * (s + u)];
+#pragma unroll
+            for (int u = 0; u < kPhaseUnroll; u++)
+#pragma unroll
+                for (int t = 0; t < T; t++)
+                    acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x[u][t], wc[u], acc[t], 0, 0, 0);
         }
-        if (s <= hi_i) {
-            const ConstDoubles wc = wp + 2 * s;
-            const float* xc = xr + s;
-            float x[8];
-            double w[16];
-#pragma unroll
-            for (int t = 0; t < 8; t++) {
-                x[t] = xc[t];
-                w[2 * t] = wc[2 * t];
-                w[2 * t + 1] = wc[2 * t + 1];
-            }
-#pragma unroll
-            for (int t = 0; t < 7; t++)
-                if (s + t <= hi_i) {
-                    a0 = fma(w[2 * t], (double)x[t], a0);
-                    a1 = fma(w[2 * t + 1], (double)x[t], a1);
-                }
-        }
-        pair_edge(xr, wp, rg, hi_i + 1, hi_u, a0, a1);
-        const long long i = i0 + q0;
-        if (i < a.out_n) outc[i] = (float)a0;
-        if (q0 + 1 < a.up && i + 1 < a.out_n) outc[i + 1] = (float)a1;
+        phase_store(a, acc, outp, left, xs + F, g, lane);
     }
 }
 
-// LDS bytes of one staged tile (zero: the tile does not fit in `budget` bytes, the device's LDS
-// per workgroup, and the per-tap kernel is used).
-int phase_lds_bytes(int down, int ntap, long long budget, int* width, int* pitch) {
-    const long long wd = (long long)down + ntap + kPhaseOverread;
-    const long long pt = wd | 1;
-    const long long bytes = kPhaseTile * pt * (long long)sizeof(float);
-    if (bytes > budget) return 0;
-    *width = (int)wd;
-    *pitch = (int)pt;
-    return (int)bytes;
-}
+// The period multiple m and the shape of the tables for a ratio up / down with ntap taps a phase.
+struct PhaseShape {
+    int m = 0, groups = 0, ks = 0, width = 0, pitch = 0;
+};
 
+// f(q) = floor(q down / up).
+inline int phase_floor(int q, int up, int down) { return (int)((long long)q * down / up); }
+
+// m: more than one period where the period alone wastes columns of its last group (U not a
+// multiple of 16) or has too few groups to give the waves of a workgroup one each (8), as long as
+// the rows stay short enough for 32 of them in half the LDS (two workgroups a CU). The cost of each
+// candidate is its padding times a factor for what it misses; the smallest m of least cost is
+// taken. m = 0: no shape fits `budget` bytes of LDS with 16 rows.
+PhaseShape phase_shape(int up, int down, int ntap, long long budget) {
+    PhaseShape best;
+    double least = 0.0;
+    for (int m = 1; m <= 128; m++) {
+        const long long U = (long long)m * up, D = (long long)m * down;
+        if (m > 1 && (U > 1024 || D > 4096)) break;
+        const int groups = (int)((U + 15) / 16);
+        int span = 0, last = 0;
+        for (int g = 0; g < groups; g++) {
+            last = phase_floor(16 * g, up, down);
+            span = std::max(span, phase_floor((int)std::min<long long>(16LL * g + 15, U - 1), up, down) - last);
+        }
+        const int ks = (ntap + span + 4 * kPhaseUnroll - 1) / (4 * kPhaseUnroll) * kPhaseUnroll;
+        const int width = last + 4 * ks, pitch = width + (6 - width % 4) % 4;   // the next 2 mod 4
+        if (16LL * pitch * 4 > budget) break;                  // rows only grow with m
+        double cost = 16.0 * groups / (double)U;
+        if (groups < 8) cost *= 1.0 + 0.05 * (8 - groups);
+        if (32LL * pitch * 4 > budget / 2) cost *= 1.15;
+        if (best.m == 0 || cost < least - 1e-9) {
+            best = PhaseShape{m, groups, ks, width, pitch};
+            least = cost;
+        }
+    }
+    return best;
+}
 
 __global__ __launch_bounds__(256) void copy_kernel(const float* __restrict__ in, float* __restrict__ out, size_t n) {
     for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (size_t)gridDim.x * 256) out[e] = in[e];
@@ -312,23 +368,23 @@ STX_API stx_status stx_resampler_create(int src_rate, int dst_rate, stx_resample
             const int up = dst_rate / g, down = src_rate / g;
             const int omin = -(int)std::floor(half), omax = (int)std::floor(half) + 1;
             const int ntap = omax - omin + 1;
-            std::vector<double> phase;
+            std::vector<double> weights;
+            std::vector<int> goff;
             std::vector<int2> range;
-            // The staged tile must fit in the device's LDS per workgroup; above 64 KB the kernel
-            // is allowed that much dynamic LDS first.
-            int width = 0, pitch = 0;
-            int lds_bytes = phase_lds_bytes(down, ntap, lds_max, &width, &pitch);
-            if (lds_bytes > 64 * 1024 &&
-                hipFuncSetAttribute((const void*)resample_phase_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    lds_max) != hipSuccess) {
+            const long long budget = lds_max - 1024;                 // beside the kernel's static LDS
+            PhaseShape shape;
+            if ((long long)up * ntap <= kPhaseMaxWeights) shape = phase_shape(up, down, ntap, budget);
+            // Above 64 KB a kernel is allowed that much dynamic LDS first.
+            auto allow = [&](const void* k) {
+                if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)budget) == hipSuccess) return true;
                 (void)hipGetLastError();
-                lds_bytes = 0;
-            }
-            std::vector<double> pair;
-            std::vector<int4> prange;
-            if ((long long)up * ntap <= kPhaseMaxWeights && lds_bytes > 0) {
-                phase.assign((size_t)up * ntap, 0.0);
-                range.assign(up, make_int2(0, -1));
+                return false;
+            };
+            if (shape.m > 0 && !(allow((const void*)resample_phase_kernel<1>) && allow((const void*)resample_phase_kernel<2>)))
+                shape.m = 0;
+            if (shape.m > 0 && (long long)shape.groups * shape.ks * 64 <= kPhaseMaxTable) {
+                std::vector<double> phase((size_t)up * ntap, 0.0);
+                std::vector<int2> taps(up, make_int2(0, -1));
                 for (int p = 0; p < up; p++) {
                     const double frac = (double)p / up;
                     int lo = ntap, hi = -1;
@@ -342,49 +398,41 @@ STX_API stx_status stx_resampler_create(int src_rate, int dst_rate, stx_resample
                         lo = std::min(lo, k);
                         hi = std::max(hi, k);
                     }
-                    range[p] = make_int2(lo, hi);
+                    taps[p] = make_int2(lo, hi);
                 }
-                // Pairs of neighbouring phases q0 = 2 jp and q1 = q0 + 1, whose taps start at
-                // floor(q down / up) + omin: q1's are d = fq1 - fq0 later, so its row goes in at
-                // s = k + d. An odd last phase is paired with itself.
-                auto fq = [&](int q) { return (int)((long long)q * down / up); };
-                const int npairs = (up + 1) / 2;
-                int dmax = 0;
-                for (int jp = 0; jp < npairs; jp++)
-                    if (2 * jp + 1 < up) dmax = std::max(dmax, fq(2 * jp + 1) - fq(2 * jp));
-                const int rs = 2 * (ntap + dmax + kPhaseOverread);
-                pair.assign((size_t)npairs * rs, 0.0);
-                prange.resize(npairs);
-                for (int jp = 0; jp < npairs; jp++) {
-                    const int q0 = 2 * jp, q1 = q0 + 1 < up ? q0 + 1 : q0;
-                    const int p0 = (int)((long long)q0 * down % up), p1 = (int)((long long)q1 * down % up);
-                    const int d = fq(q1) - fq(q0);
-                    double* row = pair.data() + (size_t)jp * rs;
-                    for (int k = range[p0].x; k <= range[p0].y; k++) row[2 * k] = phase[(size_t)p0 * ntap + k];
-                    if (q1 != q0)
-                        for (int k = range[p1].x; k <= range[p1].y; k++)
-                            row[2 * (k + d) + 1] = phase[(size_t)p1 * ntap + k];
-                    prange[jp] = make_int4(range[p0].x, range[p0].y, d + range[p1].x, d + range[p1].y);
+                const int U = shape.m * up;
+                weights.assign((size_t)shape.groups * shape.ks * 64, 0.0);
+                goff.resize(shape.groups);
+                range.resize(U);
+                for (int q = 0; q < U; q++) {
+                    const int g = q / 16, F = phase_floor(16 * g, up, down), d = phase_floor(q, up, down) - F;
+                    const int p = (int)((long long)q * down % up);
+                    goff[g] = F;
+                    range[q] = make_int2(taps[p].x + d, taps[p].y + d);
+                    double* wg = weights.data() + (size_t)g * shape.ks * 64;
+                    for (int k = taps[p].x; k <= taps[p].y; k++)
+                        wg[(k + d) / 4 * 64 + (k + d) % 4 * 16 + q % 16] = phase[(size_t)p * ntap + k];
                 }
-                r->up = up;
-                r->down = down;
+                r->U = U;
+                r->D = shape.m * down;
                 r->omin = omin;
-                r->npairs = npairs;
-                r->rs = rs;
-                r->width = width;
-                r->pitch = pitch;
-                r->lds_bytes = lds_bytes;
+                r->groups = shape.groups;
+                r->ks = shape.ks;
+                r->width = shape.width;
+                r->pitch = shape.pitch;
+                r->lds_max = budget;
             }
             hipError_t e = hipMalloc(&r->d_table, sizeof(double) * table.size());
             if (e == hipSuccess)
                 e = hipMemcpy(r->d_table, table.data(), sizeof(double) * table.size(), hipMemcpyHostToDevice);
-            if (e == hipSuccess && !pair.empty()) {
-                e = hipMalloc(&r->d_pair, sizeof(double) * pair.size());
-                if (e == hipSuccess) e = hipMalloc(&r->d_prange, sizeof(int4) * prange.size());
-                if (e == hipSuccess)
-                    e = hipMemcpy(r->d_pair, pair.data(), sizeof(double) * pair.size(), hipMemcpyHostToDevice);
-                if (e == hipSuccess)
-                    e = hipMemcpy(r->d_prange, prange.data(), sizeof(int4) * prange.size(), hipMemcpyHostToDevice);
+            auto upload = [&](auto*& d, const auto& h) {
+                if (e == hipSuccess) e = hipMalloc(&d, sizeof(h[0]) * h.size());
+                if (e == hipSuccess) e = hipMemcpy(d, h.data(), sizeof(h[0]) * h.size(), hipMemcpyHostToDevice);
+            };
+            if (!weights.empty()) {
+                upload(r->d_weights, weights);
+                upload(r->d_goff, goff);
+                upload(r->d_range, range);
             }
             if (e != hipSuccess) {
                 stx_resampler_destroy(r);
@@ -398,8 +446,9 @@ STX_API stx_status stx_resampler_create(int src_rate, int dst_rate, stx_resample
 STX_API void stx_resampler_destroy(stx_resampler* r) {
     if (!r) return;
     if (r->d_table) (void)hipFree(r->d_table);
-    if (r->d_pair) (void)hipFree(r->d_pair);
-    if (r->d_prange) (void)hipFree(r->d_prange);
+    if (r->d_weights) (void)hipFree(r->d_weights);
+    if (r->d_goff) (void)hipFree(r->d_goff);
+    if (r->d_range) (void)hipFree(r->d_range);
     delete r;
 }
 
@@ -432,14 +481,22 @@ STX_API stx_status stx_resample(const stx_resampler* r, const float* in, int cha
         // The phase table unless STX_RESAMPLE_EXACT=1 (read at each call) asks for the per-tap
         // kernel, which gives the reference's bits.
         const char* exact = std::getenv("STX_RESAMPLE_EXACT");
-        if (r->d_pair && !(exact && exact[0] == '1')) {
-            PhaseArgs pa{in, out, r->d_pair, r->d_prange, n, out_n, r->up, r->down, r->omin, r->npairs, r->rs, r->width, r->pitch,
-                         FastDiv((unsigned)r->up)};
-            const long long groups = (out_n + r->up - 1) / r->up;                // output groups M
-            STX_REQUIRE(channels < 65536, "too many channels");
-            const long long tiles = (groups + kPhaseTile - 1) / kPhaseTile;
-            const dim3 pg((unsigned)tiles, (unsigned)channels);
-            hipLaunchKernelGGL(resample_phase_kernel, pg, dim3(kPhaseWaves * 64), (unsigned)r->lds_bytes, s, pa);
+        if (r->d_weights && !(exact && exact[0] == '1')) {
+            const PhaseArgs pa{in, out, r->d_weights, r->d_goff, r->d_range, n, out_n, r->U, r->D, r->omin, r->groups,
+                               r->ks, r->width, r->pitch};
+            const long long periods = (out_n + r->U - 1) / r->U;
+            const int waves = std::min(r->groups, kPhaseMaxWaves);
+            auto go = [&](auto tiles) {
+                constexpr int T = decltype(tiles)::value;
+                const dim3 grid((unsigned)((periods + 16 * T - 1) / (16 * T)), (unsigned)channels);
+                hipLaunchKernelGGL(resample_phase_kernel<T>, grid, dim3(waves * 64), (unsigned)(16 * T * r->pitch * 4), s, pa);
+            };
+            // Two tiles of 16 periods where their rows leave room for two workgroups a CU and there
+            // are two workgroups for each CU of the device (a weight operand then feeds two products).
+            if (32LL * r->pitch * 4 <= r->lds_max / 2 && (periods + 31) / 32 * channels >= 2LL * device_cus())
+                go(std::integral_constant<int, 2>{});
+            else
+                go(std::integral_constant<int, 1>{});
             launch_check("resample_phase_kernel");
             return;
         }

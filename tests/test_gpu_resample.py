@@ -4,8 +4,8 @@ Bars: the per-tap kernel (STX_RESAMPLE_EXACT=1) is bit-exact (the device sums th
 double products in the reference's order over a table computed by the reference's formula);
 the default phase-table kernel, whose weights come from the output's exact rational position
 instead of the reference's rounded one, has SNR >= 110 dB and every sample within 1e-6 of the
-output's rms. A rate pair whose staged input tile exceeds the device's LDS per workgroup
-(44.1 -> 8 kHz here: 210 KB) takes the per-tap kernel by default and is bit-exact either way.
+output's rms. A rate pair with more than 2^18 phase weights (44,100 -> 44,101 Hz here) takes the
+per-tap kernel by default and is bit-exact either way.
 Shapes: a 180 s stereo song at 48 kHz to the models' 44.1 kHz, and short inputs for other rate
 pairs, mono, stereo and 3 channels.
 """
@@ -62,8 +62,8 @@ def test_resample_parity(device, rs, src, dst, C, n, monkeypatch):
                                          (96000, 44100, 3, 9601)])
 def test_resample_nonfinite(device, rs, src, dst, C, n, monkeypatch):
     """NaN, +inf and -inf samples (NaN at each end) reach exactly the outputs whose window holds
-    them in the reference (src/audio.h:44-52): the phase kernel's pair loop sums a tap only where
-    its own phase's window has it, so the NaN and infinite outputs are the oracle's and the finite
+    them in the reference (src/audio.h:44-52): where a sum is not finite the phase kernel sums again, each
+    output over its own phase's taps, so the NaN and infinite outputs are the oracle's and the finite
     outputs keep the usual bound; the per-tap kernel is bit-identical, NaNs included.
 
     An infinite output's sign is its tap's weight's. At a zero of the kernel the reference's weight
@@ -87,6 +87,33 @@ def test_resample_nonfinite(device, rs, src, dst, C, n, monkeypatch):
     assert float(np.max(np.abs(got[fin].astype(np.float64) - want[fin]))) <= 1e-6 * rms
     monkeypatch.setenv("STX_RESAMPLE_EXACT", "1")
     assert np.array_equal(host(r(xd)), want, equal_nan=True)
+
+
+# Ratios of one phase (the period repeated up to 128 times) and of many, groups of 16 phases that end inside a
+# period (147, 441), windows from 72 to 836 samples; lengths from one sample through the ends of tiles of 16 and
+# 32 periods, and one launch of two tiles a wave (8 channels of half a million samples).
+@pytest.mark.parametrize("src,dst,C,n", [(48000, 16000, 2, 70001), (88200, 44100, 1, 5000), (44100, 88200, 2, 16 * 64 + 1),
+                                         (32000, 44100, 1, 32 * 320 - 1), (96000, 8000, 2, 30011), (8000, 96000, 1, 2049),
+                                         (11025, 48000, 3, 16 * 147), (48000, 44100, 8, 500001), (44100, 48000, 1, 16 * 147 + 1),
+                                         (48000, 32000, 1, 1), (96000, 8000, 1, 13), (44100, 44101, 1, 3001)])
+def test_resample_ratios(device, rs, src, dst, C, n):
+    """The default kernel against the oracle, within the bounds of test_resample_parity; then with a NaN, an infinity
+    and a -infinity, which reach exactly the outputs whose windows hold them."""
+    x = synth.normal(src % 997 + n % 89, (C, n), 0.3)
+    r = stx.Resampler(src, dst)
+    want = rs(x, src, dst)
+    got = host(r(dev(x, device)))
+    assert got.shape == want.shape
+    rms = max(float(np.sqrt(np.mean(want.astype(np.float64) ** 2))), 1e-3) if want.size else 1.0
+    assert float(np.max(np.abs(got.astype(np.float64) - want), initial=0.0)) <= 1e-6 * rms
+    if n < 2000 or C > 3:
+        return
+    x[0, n // 3], x[-1, n // 2], x[-1, n - 1] = np.inf, -np.inf, np.nan
+    want = rs(x, src, dst)
+    got = host(r(dev(x, device)))
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    fin = np.isfinite(want)
+    assert float(np.max(np.abs(got[fin].astype(np.float64) - want[fin]))) <= 1e-6 * rms
 
 
 def test_equal_rates_copy(device):
