@@ -610,4 +610,120 @@ inline bool mixed_plan_is(const MixedRadix& p, const int* radix, int count) {
     return true;
 }
 
+// ------------------------------------------------------ several mixed-radix frames a workgroup
+// The passes in place: TPF threads hold all of a frame's points of one pass in registers (at most
+// 16 a thread and butterfly count below) between its reads and its writes, so one LDS buffer a frame
+// is enough where mixed_fft ping-pongs between two, and twice the frames fit a CU. A frame of
+// TPF <= 64 threads lies in one wave, whose LDS accesses are performed in order: no barriers.
+template <int TPF>
+__device__ __forceinline__ void frame_sync() {
+    if constexpr (TPF <= 64) wave_lds_sync();
+    else lds_barrier();
+}
+
+// W_n^m: one LDS read of the full table (small n: also one rounding instead of three), or the
+// two-level table's product (mixed_tw).
+struct TwFull {
+    const float2* t;
+    __device__ __forceinline__ float2 operator()(int m) const { return t[m]; }
+};
+struct TwTwoLevel {
+    const float2* t;
+    __device__ __forceinline__ float2 operator()(int m) const { return mixed_tw(t, m); }
+};
+
+// One pass of radix R after sub-transforms of length Ns (see mixed_pass), in place in buf, by the
+// TPF threads of a frame; M <= 16 TPF, so a thread takes at most ceil(16 / R) butterflies (15: one,
+// the host checks M <= 15 TPF). MC, NSC: M and Ns where they are compile-time constants, else 0.
+template <int R, int TPF, int MC, int NSC, class TW>
+__device__ __forceinline__ void frame_pass(float2* buf, int M_rt, int Ns_rt, int scale, const TW& tw, int j) {
+    const int M = MC ? MC : M_rt, Ns = NSC ? NSC : Ns_rt;
+    constexpr int IT = R == 15 ? 1 : (16 + R - 1) / R;
+    const int B = M / R;
+    const unsigned inv = Ns > 1 ? 0xffffffffu / (unsigned)Ns + 1u : 0u;
+    float2 v[IT][R];
+    int k[IT], base[IT];
+#pragma unroll
+    for (int it = 0; it < IT; it++) {
+        const int b = min(j + it * TPF, B - 1);
+        const int blk = NSC ? b / Ns : Ns > 1 ? (int)__umulhi((unsigned)b, inv) : b;
+        k[it] = b - blk * Ns;
+        base[it] = blk * Ns * R + k[it];
+#pragma unroll
+        for (int r = 0; r < R; r++) v[it][r] = buf[mixed_pad(b + r * B)];
+    }
+    frame_sync<TPF>();
+#pragma unroll
+    for (int it = 0; it < IT; it++) {
+        if (j + it * TPF < B) {
+            if (Ns > 1) {
+#pragma unroll
+                for (int r = 1; r < R; r++) {
+                    v[it][r] = cmul(v[it][r], tw(k[it] * r * scale));
+                    // A few twiddles in registers at a time (at 128 registers all 15 spill).
+                    if (R > 8 && r % 5 == 0) __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            Dft<R>::run(v[it]);
+#pragma unroll
+            for (int r = 0; r < R; r++) buf[mixed_pad(base[it] + r * Ns)] = v[it][r];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    frame_sync<TPF>();
+}
+
+// The passes of plan p from pass `first` on (Ns: the product of the radices before it).
+template <int TPF, class TW>
+__device__ __forceinline__ void frame_passes(float2* buf, int M, const MixedRadix& p, int first, int Ns, int tw_mul, const TW& tw,
+                                             int j) {
+    for (int i = first; i < p.count; i++) {
+        // Opaque copies: the passes' LDS offsets, which depend on j and M only, are computed where
+        // they are used instead of being held for every radix across the loop.
+        int jj = j, m = M;
+        asm volatile("" : "+v"(jj), "+s"(m));
+        const int R = p.r[i];
+        const int scale = (m / (Ns * R)) * tw_mul;
+        switch (R) {
+            case 16: frame_pass<16, TPF, 0, 0>(buf, m, Ns, scale, tw, jj); break;
+            case 8: frame_pass<8, TPF, 0, 0>(buf, m, Ns, scale, tw, jj); break;
+            case 4: frame_pass<4, TPF, 0, 0>(buf, m, Ns, scale, tw, jj); break;
+            case 2: frame_pass<2, TPF, 0, 0>(buf, m, Ns, scale, tw, jj); break;
+            case 15: frame_pass<15, TPF, 0, 0>(buf, m, Ns, scale, tw, jj); break;
+            case 3: frame_pass<3, TPF, 0, 0>(buf, m, Ns, scale, tw, jj); break;
+            default: frame_pass<5, TPF, 0, 0>(buf, m, Ns, scale, tw, jj); break;
+        }
+        Ns *= R;
+    }
+}
+
+// The same for a plan known at compile time (radices R, Rest... after sub-transforms of length Ns).
+template <int TPF, int M, int TWMUL, int Ns, int R, int... Rest, class TW>
+__device__ __forceinline__ void frame_passes_ct(float2* buf, const TW& tw, int j) {
+    frame_pass<R, TPF, M, Ns>(buf, M, Ns, (M / (Ns * R)) * TWMUL, tw, j);
+    if constexpr (sizeof...(Rest) > 0) frame_passes_ct<TPF, M, TWMUL, Ns * R, Rest...>(buf, tw, j);
+}
+
+// The first pass of a plan that starts with radix 16, from registers: v holds elements
+// j + r M / 16 of the threads j < M / 16.
+template <int TPF>
+__device__ __forceinline__ void frame_first16(float2 (&v)[16], float2* buf, int M, int j) {
+    if (j < M / 16) {
+        Dft<16>::run(v);
+#pragma unroll
+        for (int r = 0; r < 16; r++) buf[j * 17 + r] = v[r];
+    }
+    frame_sync<TPF>();
+}
+
+// Threads per frame for an M-point plan: the smallest that holds a pass in 16 points a thread, 0
+// where none of the built ones (16 .. 256) does.
+inline int frame_threads(int M, const MixedRadix& p) {
+    bool r15 = false;
+    for (int i = 0; i < p.count; i++) r15 = r15 || p.r[i] == 15;
+    for (int t = 16; t <= 256; t *= 2)
+        if (M <= (r15 ? 15 : 16) * t) return t;
+    return 0;
+}
+
 }  // namespace stx

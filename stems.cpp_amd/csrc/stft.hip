@@ -18,10 +18,11 @@
 //         frame that overlaps it (frames shared by two tiles are transformed by both), sums the
 //         windowed frames in frame order in registers and divides by the window-squared
 //         envelope, evaluated in closed form per sample;
-//       - two kernels (the mixed-radix sizes, with a workspace of C*T*N floats): one
-//         inverse-transforms each frame once and writes it windowed to the workspace, the
-//         next sums and divides. Power-of-two sizes run the fused kernel with or without a
-//         workspace (measured faster at every size).
+//       - two kernels (the mixed-radix sizes with a large n or few frames, with a workspace of
+//         C*T*N floats): one inverse-transforms each frame once and writes it windowed to the
+//         workspace, the next sums and divides. Power-of-two sizes run the fused kernel with or
+//         without a workspace (measured faster at every size), mixed-radix calls with many frames
+//         of n <= 2048 a fused one of their own (istft_tile_kernel).
 #include <algorithm>
 #include <type_traits>
 #include <memory>
@@ -603,7 +604,7 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_kernel(IstftArgs a) 
 // Bluestein (three power-of-two transforms of at least 2n - 1 points); here one workgroup runs
 // the n/2-point transform of a real frame directly, radix 16 / 8 / 4 / 2 / 15 / 3 / 5 Stockham passes
 // ping-ponging between two LDS buffers with twiddles W_n^m from a table computed in double.
-// Frames are packed and split as in the power-of-two kernels; the iSTFT always takes the
+// Frames are packed and split as in the power-of-two kernels; the iSTFT takes the
 // two-kernel path (frames to the workspace, then istft_ola_kernel). One frame per workgroup,
 // numbered XCD-aware (xcd_block): consecutive frames run on one XCD, so the F-major spectrum's
 // rows, where each frame owns 8 bytes of a 128-byte line, are written (or read) through one L2
@@ -779,6 +780,202 @@ __global__ __launch_bounds__(kMixedThreads * FPB) void istft_frames_mixed_kernel
             store_stream(dst + 2 * i, o.x);
             store_stream(dst + 2 * i + 1, o.y);
         }
+    }
+}
+
+// ---------------------------------------------- mixed-radix sizes, several frames a workgroup
+// TPF threads a frame and JOBS neighbouring frames a workgroup, transformed in place (frame_pass): the
+// half transform of n_fft 960 has 480 points, 30 radix-16 butterflies, so a workgroup of 512 threads per
+// frame (stft_mixed_kernel) left 94 % of them idle, and in the f-major layout each frame owns 8
+// bytes of a row; JOBS = 16 frames make runs of 128. With TPF <= 64 a frame is one wave's, so its
+// passes need no barrier. The twiddles are the full table of W_n^m in LDS for n <= 2048. Bound by LDS
+// traffic and VALU issue: n_fft 960, hop 480, a minute of stereo f-major 120 -> 24.9 us (3.4 TB/s of the
+// signal and the spectrum), iSTFT 143 -> 37.9; n_fft 320, hop 80, 12,502 frames 95 -> 15.3 and 109 -> 19.3.
+constexpr int kFrameTw = 2048;                         // full tables up to this n
+
+// Dynamic LDS: JOBS slots of frame_slot(M) float2, then the twiddles, then (iSTFT) the window.
+// Odd slots: the JOBS frames of one bin lie in different banks.
+__host__ __device__ constexpr int frame_slot(int M) { return mixed_padded(M) | 1; }
+
+// Copies cnt <= COUNT elements to LDS in two halves, as Staged.
+template <int COUNT, int NT, class T>
+struct StagedRt {
+    static constexpr int R = (COUNT + NT - 1) / NT;
+    T v[R];
+    __device__ __forceinline__ void load(const T* __restrict__ src, int cnt, int tid) {
+#pragma unroll
+        for (int r = 0; r < R; r++) v[r] = src[min(tid + r * NT, cnt - 1)];
+    }
+    __device__ __forceinline__ void store(T* dst, int cnt, int tid) const {
+#pragma unroll
+        for (int r = 0; r < R; r++)
+            if (tid + r * NT < cnt) dst[tid + r * NT] = v[r];
+    }
+};
+
+template <int TPF, int JOBS>
+__global__ __launch_bounds__(TPF * JOBS) __attribute__((amdgpu_waves_per_eu(4))) void stft_frames_kernel(StftArgs a, MixedRadix p, const float2* __restrict__ twn, int n,
+                                                                 FastDiv ft) {
+    extern __shared__ float2 sm[];
+    constexpr int NT = TPF * JOBS;
+    const int M = n / 2, slot = frame_slot(M);
+    const int lb = xcd_block();
+    if (lb >= a.nblocks) return;                       // whole block idle: no barrier reached
+    const int tid = (int)threadIdx.x, g = tid / TPF, j = tid % TPF;
+    float2* buf = sm + g * slot;
+    float2* twl = sm + JOBS * slot;
+    StagedRt<kFrameTw, NT, float2> tws;
+    tws.load(twn, n, tid);
+    const int f0 = lb * JOBS, f = min(f0 + g, a.jobs - 1);      // past the end: the last frame again, not written
+    const int c = (int)ft.div((unsigned)f), t = f - c * a.T;
+    const float* xc = a.x + (size_t)c * a.len;
+    const int m0 = a.frame0 + t * a.hop;
+    const int base = m0 - M - a.pre_left;              // its signal index when nothing reflects
+    const bool interior = base >= 0 && base + n <= a.len;
+    // Elements j + u step: the first pass's own order when it is a radix-16 one (straight from the
+    // registers), else one after the other.
+    const bool first16 = p.r[0] == 16;
+    const int step = first16 ? M / 16 : TPF;
+    const float2* win2 = reinterpret_cast<const float2*>(a.win);
+    float2 v[16];
+    auto element = [&](int u) { return min(j + u * step, M - 1); };
+    if (interior) {
+#pragma unroll
+        for (int u = 0; u < 16; u++) {
+            const float* xs = xc + base + 2 * element(u);
+            v[u] = make_float2(xs[0], xs[1]);
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < 16; u++) {
+            const int e = element(u);
+            v[u] = make_float2(xc[padded_index_rt(m0 + 2 * e, a, n)], xc[padded_index_rt(m0 + 2 * e + 1, a, n)]);
+            if (u % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // few frames: not all the index registers at once
+        }
+    }
+    float2 w[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) w[u] = win2[element(u)];
+#pragma unroll
+    for (int u = 0; u < 16; u++) v[u] = make_float2(v[u].x * w[u].x, v[u].y * w[u].y);
+    tws.store(twl, n, tid);
+    if (first16) {
+        frame_first16<TPF>(v, buf, M, j);
+    } else {
+#pragma unroll
+        for (int u = 0; u < 16; u++)
+            if (j + u * TPF < M) buf[mixed_pad(j + u * TPF)] = v[u];
+    }
+    __syncthreads();                                   // the twiddles
+    frame_passes<TPF>(buf, M, p, first16 ? 1 : 0, first16 ? 16 : 1, 2, TwFull{twl}, j);
+    // X[k] = E[k] + W_n^k O[k], k <= n/2, as in stft_kernel.
+    const float hs = 0.5f * a.scale;
+    auto bin = [&](const float2* z, int k) {
+        const float2 zk = z[mixed_pad(k == M ? 0 : k)], zm = z[mixed_pad(k == 0 ? 0 : M - k)], w = twl[k];
+        const float er = zk.x + zm.x, ei = zk.y - zm.y;
+        const float orr = zk.y + zm.y, oi = zm.x - zk.x;
+        return make_float2((er + w.x * orr - w.y * oi) * hs, (ei + w.x * oi + w.y * orr) * hs);
+    };
+    if (a.layout == STX_SPEC_F_MAJOR) {
+        __syncthreads();                               // every frame of the block
+        const int gg = tid % JOBS, ff = f0 + gg;
+        if (ff >= a.jobs) return;
+        const int cc = (int)ft.div((unsigned)ff), tt = ff - cc * a.T;
+        const float2* z = sm + gg * slot;
+        float2* col = a.spec + (size_t)cc * a.F * a.T + tt;
+        for (int k = tid / JOBS; k < a.F; k += TPF) col[(size_t)k * a.T] = bin(z, k);
+    } else if (f0 + g < a.jobs) {
+        float2* row = a.spec + ((size_t)c * a.T + t) * a.F;
+        for (int k = j; k < a.F; k += TPF) store_stream(row + k, bin(buf, k));
+    }
+}
+
+// The iSTFT of the same sizes with the overlap-add in the workgroup, as istft_kernel's: a tile of
+// output samples, the at most JOBS frames that overlap it (frames shared by two tiles are transformed
+// by both), the sums over them in frame order and the quotient by the window-squared envelope. No
+// frame goes through memory.
+template <int TPF, int JOBS>
+__global__ __launch_bounds__(TPF * JOBS) __attribute__((amdgpu_waves_per_eu(4))) void istft_tile_kernel(IstftArgs a, MixedRadix p, const float2* __restrict__ twn, int n,
+                                                                FastDiv fhop, FastDiv ftiles) {
+    extern __shared__ float2 sm[];
+    constexpr int NT = TPF * JOBS;
+    const int M = n / 2, slot = frame_slot(M);
+    const int lb = xcd_block();
+    if (lb >= a.nblocks) return;                       // whole block idle: no barrier reached
+    const int tid = (int)threadIdx.x, g = tid / TPF, j = tid % TPF;
+    float2* buf = sm + g * slot;
+    float2* twl = sm + JOBS * slot;
+    float* win = reinterpret_cast<float*>(twl + n);
+    StagedRt<kFrameTw, NT, float2> tws;
+    StagedRt<kFrameTw, NT, float> wins;
+    tws.load(twn, n, tid);
+    wins.load(a.win, n, tid);
+    const int c = (int)ftiles.div((unsigned)lb), tile = lb - c * a.tiles;
+    const int J0 = max(a.out_off, a.tile_origin + tile * a.tile_len);
+    const int J1 = min(a.out_off + a.out_len, a.tile_origin + (tile + 1) * a.tile_len);
+    const int st_lo = max(0, max(0, ceildiv(J0 - n + 1, a.hop)) - a.frame_off);
+    const int st_hi = min(a.T - 1, floordiv(J1 - 1, a.hop) - a.frame_off);
+    const float2* sc = a.spec + (size_t)c * a.T * a.F;
+    if (st_lo <= st_hi) {                              // uniform
+        // Bins 0..M of every frame (past st_hi: frame st_hi again, never summed), neighbouring
+        // lanes on neighbouring addresses in either layout, every load before the first LDS write.
+        float2 x[17];
+        if (a.layout == STX_SPEC_F_MAJOR) {
+            const float2* col = sc + min(st_lo + tid % JOBS, st_hi);
+#pragma unroll
+            for (int i = 0; i < 17; i++) x[i] = col[(size_t)min(tid / JOBS + i * TPF, min(M, a.F - 1)) * a.T];
+        } else {
+            const float2* row = sc + (size_t)min(st_lo + g, st_hi) * a.F;
+#pragma unroll
+            for (int i = 0; i < 17; i++) x[i] = row[min(j + i * TPF, min(M, a.F - 1))];
+        }
+        tws.store(twl, n, tid);
+        wins.store(win, n, tid);
+        const bool fm = a.layout == STX_SPEC_F_MAJOR;
+        float2* xs = sm + (fm ? tid % JOBS : g) * slot;
+        const int k0 = fm ? tid / JOBS : j;
+#pragma unroll
+        for (int i = 0; i < 17; i++)
+            if (k0 + i * TPF <= M) xs[mixed_pad(k0 + i * TPF)] = x[i];
+        __syncthreads();
+        const bool first16 = p.r[0] == 16;
+        const int step = first16 ? M / 16 : TPF;
+        float2 v[16];
+#pragma unroll
+        for (int u = 0; u < 16; u++) {
+            const int k = min(j + u * step, M - 1);
+            v[u] = inverse_split_w(buf[mixed_pad(k)], buf[mixed_pad(M - k)], k, a.keep_nyquist, twl[k]);
+        }
+        frame_sync<TPF>();                             // the bins read before the transform overwrites them
+        if (first16) {
+            frame_first16<TPF>(v, buf, M, j);
+        } else {
+#pragma unroll
+            for (int u = 0; u < 16; u++)
+                if (j + u * TPF < M) buf[mixed_pad(j + u * TPF)] = v[u];
+            frame_sync<TPF>();
+        }
+        frame_passes<TPF>(buf, M, p, first16 ? 1 : 0, first16 ? 16 : 1, 2, TwFull{twl}, j);
+    } else {
+        wins.store(win, n, tid);
+    }
+    __syncthreads();
+    // Samples of frame st are z = conj(fft): 2i (real) and 2i + 1 (minus imaginary) of element i.
+    const int hop = a.hop, K0 = (n - 1) / hop, rK = n - 1 - K0 * hop;
+    float* oc = a.out + (size_t)c * a.out_len;
+    for (int J = J0 + tid; J < J1; J += NT) {
+        const int A = (int)fhop.div((unsigned)J), R = J - A * hop, K = R <= rK ? K0 : K0 - 1;
+        float sum = 0.f, env = 0.f;
+        for (int q = K; q >= 0; q--) {                 // frame order
+            const int tf = A - q, st = tf - a.frame_off, pos = R + q * hop;
+            const float w = win[pos];
+            if (tf >= 0 && tf < a.env_frames) env += w * w;
+            if (st >= st_lo && st <= st_hi) {
+                const float2 z = sm[(st - st_lo) * slot + mixed_pad(pos >> 1)];
+                sum += ((pos & 1) ? -z.y : z.x) * w * a.norm;
+            }
+        }
+        store_stream(oc + (J - a.out_off), J < a.valid_end && env > 1e-11f ? sum / env : 0.f);
     }
 }
 
@@ -979,6 +1176,69 @@ void launch_istft_fused(IstftArgs a, int channels, hipStream_t s) {
     launch_istft_fused_jobs<N, JOBS, true>(a, channels, s);
 }
 
+// The several-frames kernels' workgroups: 16 frames of frame_threads() threads. 0: not for this plan or
+// this many frames (channels times frames): below about 1,024 they leave CUs idle and one frame a
+// workgroup is faster (n_fft 960, 368 frames: 8.7 against 9.6 us, iSTFT 11.9 against 13.6; 11,026
+// frames: 120 against 24.9, iSTFT 143 against 37.9).
+constexpr int kFrameJobs = 16;
+constexpr int kFrameMinJobs = 1024;
+int frames_plan(const stx_fft* f, long long jobs) {
+    if (jobs < kFrameMinJobs) return 0;
+    const int t = f->n <= kFrameTw ? frame_threads(f->n / 2, f->half) : 0;
+    return t <= 64 ? t : 0;
+}
+
+// Calls go(integral_constant<int, TPF>) for t = 16, 32 or 64.
+template <class F>
+void pick_frame_threads(int t, F&& go) {
+    using std::integral_constant;
+    if (t == 16) go(integral_constant<int, 16>{});
+    else if (t == 32) go(integral_constant<int, 32>{});
+    else go(integral_constant<int, 64>{});
+}
+size_t stft_frames_lds(int n) { return sizeof(float2) * ((size_t)kFrameJobs * frame_slot(n / 2) + n); }
+size_t istft_tile_lds(int n) { return stft_frames_lds(n) + sizeof(float) * n; }
+
+// Allows the kernels of this plan the CU's whole LDS (when the plan is created; the largest mixed-radix
+// n up to kFrameTw, 2000, takes 156.3 KB).
+void allow_frames_lds(const stx_fft* f) {
+    if (istft_tile_lds(f->n) <= 64 * 1024 || !frames_plan(f, kFrameMinJobs)) return;
+    pick_frame_threads(frames_plan(f, kFrameMinJobs), [&](auto tpf) {
+        constexpr int TPF = decltype(tpf)::value;
+        const void* ks[2] = {reinterpret_cast<const void*>(stft_frames_kernel<TPF, kFrameJobs>),
+                             reinterpret_cast<const void*>(istft_tile_kernel<TPF, kFrameJobs>)};
+        for (const void* k : ks)
+            hip_check(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024), "hipFuncSetAttribute");
+    });
+}
+
+void launch_stft_frames(const stx_fft* f, StftArgs a, hipStream_t s) {
+    a.nblocks = (a.jobs + kFrameJobs - 1) / kFrameJobs;
+    const size_t lds = stft_frames_lds(f->n);
+    pick_frame_threads(frames_plan(f, a.jobs), [&](auto tpf) {
+        constexpr int TPF = decltype(tpf)::value;
+        hipLaunchKernelGGL((stft_frames_kernel<TPF, kFrameJobs>), dim3(xcd_grid(a.nblocks)), dim3(TPF * kFrameJobs), lds, s, a,
+                           f->half, f->twn, f->n, FastDiv((unsigned)a.T));
+    });
+    launch_check("stft_frames_kernel");
+}
+
+// Tiles of m hops need m + ceil(n / hop) - 1 frames: m from the block's 16 frames.
+void launch_istft_tiles(const stx_fft* f, IstftArgs a, int channels, hipStream_t s) {
+    const int span = (f->n + a.hop - 1) / a.hop, m = kFrameJobs - span + 1;
+    a.tile_len = m * a.hop;
+    a.tile_origin = a.out_off - a.out_off % a.hop;
+    a.tiles = (int)(((long long)a.out_off + a.out_len - a.tile_origin + a.tile_len - 1) / a.tile_len);
+    a.nblocks = a.tiles * channels;
+    const size_t lds = istft_tile_lds(f->n);
+    pick_frame_threads(frames_plan(f, (long long)channels * a.T), [&](auto tpf) {
+        constexpr int TPF = decltype(tpf)::value;
+        hipLaunchKernelGGL((istft_tile_kernel<TPF, kFrameJobs>), dim3(xcd_grid(a.nblocks)), dim3(TPF * kFrameJobs), lds, s, a,
+                           f->half, f->twn, f->n, FastDiv((unsigned)a.hop), FastDiv((unsigned)a.tiles));
+    });
+    launch_check("istft_tile_kernel");
+}
+
 template <int N>
 void launch_fft(float2* data, int batch, int inverse, const float2* twt, hipStream_t s) {
     constexpr int P = N >= 16 ? 16 : 8;
@@ -1049,6 +1309,11 @@ void run_istft(const stx_fft* f, IstftArgs a, int channels, void* workspace, siz
         const size_t need = istft_workspace_bytes(f->n, channels, a.T);
         STX_REQUIRE(ws_bytes >= need, "workspace too small: %zu bytes, need %zu", ws_bytes, need);
         check_extent((long long)channels * a.T * f->n, "workspace");
+        // At most half of a tile's frames shared with the next: the fused tiles.
+        if (frames_plan(f, (long long)channels * a.T) && 2 * ((f->n + a.hop - 1) / a.hop) <= kFrameJobs) {
+            launch_istft_tiles(f, a, channels, s);
+            return;
+        }
         a.frames = static_cast<float*>(workspace);
         const int jobs = channels * a.T;
         // Two frames per block where a bin's two frames are one aligned 16-byte load (f-major, T
@@ -1278,7 +1543,9 @@ STX_API stx_status stx_fft_create_any(int n, stx_fft** out) {
             stx_fft_destroy(f);
             hip_check(e, "stx_fft_create_any");
         }
-        *out = f;
+        std::unique_ptr<stx_fft, void (*)(stx_fft*)> owner(f, stx_fft_destroy);
+        allow_frames_lds(f);
+        *out = owner.release();
     });
 }
 
@@ -1394,6 +1661,10 @@ STX_API stx_status stx_torch_stft(const stx_fft* f, const float* x, int channels
         a.win_hs = f->win_hs ? f->win_hs + (normalized ? n : 0) : nullptr;
         check_extent((long long)channels * a.T * a.F, "spectrum");
         check_extent((long long)channels * len + n, "signal");
+        if (f->mixed && frames_plan(f, a.jobs)) {
+            launch_stft_frames(f, a, as_stream(stream));
+            return;
+        }
         if (f->mixed) {
             // Two frames per block where a bin row's two values are one aligned 16-byte store
             // (f-major, T even) and both frames' buffers fit in LDS (n / 2 <= 4096).

@@ -421,6 +421,39 @@ def test_mixed_pairs_unaligned_spectrum(device, n, hop, frames):
     assert np.array_equal(ya, yb)
 
 
+# n_fft with 8 .. 1,024 points in the half transform (16, 32 and 64 threads a frame, plans that start with radix 16
+# and not, the limits 240 | 250, 480 | 486, 960 | 1,000), hops from n / 8 to n, ends inside a tile of 16 frames,
+# tiles and workgroups that cross channels, and frames just below and above the switch to them (1,024).
+FRAME_CASES = [(960, 480, 3, 1023 * 160 + 7), (320, 80, 2, 80 * 600 + 3), (320, 106, 1, 106 * 1024), (480, 60, 2, 60 * 700 + 59),
+               (500, 125, 2, 125 * 530), (972, 243, 2, 243 * 520 + 1), (18, 9, 2, 9 * 900 + 4), (48, 48, 1, 48 * 1100),
+               (640, 640, 2, 640 * 520), (1536, 512, 3, 512 * 400 + 100), (1920, 480, 2, 480 * 515), (2000, 500, 2, 500 * 512),
+               (2000, 250, 4, 250 * 256), (960, 240, 1, 240 * 1022), (960, 240, 1, 240 * 1023), (960, 100, 2, 100 * 520)]
+
+
+@pytest.mark.parametrize("n,hop,channels,length", FRAME_CASES)
+@pytest.mark.parametrize("layout", [stx.F_MAJOR, stx.T_MAJOR])
+def test_mixed_many_frames(device, orc, n, hop, channels, length, layout):
+    """Mixed-radix STFT and iSTFT of calls with many frames (16 frames a workgroup) against the oracle."""
+    x = synth.normal(n + hop, (channels, length), 0.3)
+    f = any_plan(n)
+    T = length // hop + 1
+    spec = stx.torch_stft(f, to_dev(x, device), hop, layout=layout)
+    ws = stx.workspace(stx.istft_workspace_size(f, channels, T), device)
+    y = host(stx.torch_istft(f, spec, hop, layout=layout, workspace=ws))
+    spec_h = host(spec)
+    if layout == stx.T_MAJOR:
+        spec_h = spec_h.transpose(0, 2, 1)
+    w = 0.5 - 0.5 * np.cos(2.0 * np.pi * np.arange(n) / n)
+    env = np.array([np.sum(w[r::hop] ** 2) for r in range(hop)])
+    env = env[env > 1e-11]
+    for c in {0, channels - 1}:
+        ref = orc.torch_stft(x[c], n, hop)
+        assert snr_db(spec_h[c], ref) >= SNR_DB
+        # A sample is sum(w x) / sum(w^2) over the frames that cover it, so errors of variance s^2 in the frames
+        # leave s^2 / sum(w^2): hops near n, whose frames meet where their windows are small, lose that much.
+        assert snr_db(y[c], orc.torch_istft(ref, n, hop)) >= SNR_DB - max(0.0, 10.0 * np.log10(np.mean(1.0 / env)))
+
+
 def test_any_size_errors(device):
     import torch
     for n in (7, 14, 22, 20000):
