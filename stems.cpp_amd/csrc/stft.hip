@@ -254,7 +254,6 @@ struct IstftArgs {
     int tiles;               // fused: tiles per channel
     int jobs;                // two-kernel: channels * T
     int nblocks;             // fused: tiles over all channels
-    int grid;                // fused: workgroups launched (a multiple of the XCD count)
     float norm;
 };
 
@@ -342,23 +341,105 @@ __global__ __launch_bounds__(256) void istft_ola_kernel(IstftArgs a, int N) {
     store_stream(a.out + (size_t)c * a.out_len + i, y);
 }
 
+// LDS float2 of a frame's slot: KPW float2 apart modulo 32 (256 bytes of banks), since the f-major
+// staging's lanes write bin tr / JOBS of slot tr % JOBS, KPW = ceil(64 / JOBS) bins per wave, so the
+// JOBS slots' runs fall on different banks (with slots a multiple of 32 float2 apart they shared them:
+// 5x the LDS bank-conflict cycles of the t-major staging at c1). Short slots: as is.
+template <int N, int P, int JOBS>
+constexpr int istft_slot() {
+    constexpr int padn = FftCfg<N / 2, P, N>::PADN, kpw = (64 + JOBS - 1) / JOBS;
+    return padn < 512 ? padn : padn + ((kpw - padn % 32) % 32 + 32) % 32;
+}
+
+// X[0..M] of frames s0 .. s0 + JOBS - 1 into registers and on to the slots, neighbouring lanes on
+// neighbouring addresses in either layout: bins k < M are P per thread (M * JOBS = P * NT), the
+// Nyquist bins one per slot; frames outside [0, last] read the nearest one inside (finite values,
+// transformed but never summed). F-major: element e = tr + i*NT is slot e % JOBS = tr % JOBS, bin
+// tr / JOBS + i*TPJ. T-major: thread jr of a slot takes bins jr + i*TPJ of the slot's frame, the
+// FFT's own element order (one row address, then constant offsets), and the Nyquist bin.
+template <int N, int P, int JOBS, int SLOT>
+struct SpecStage {
+    static constexpr int M = N / 2, TPJ = M / P;
+    const IstftArgs& a;
+    const float2* sc;
+    float2* lds;
+    int last;
+    __device__ __forceinline__ int frame(int s) const { return min(max(s, 0), last); }
+    __device__ __forceinline__ void load(int s0, int tr, int jr, float2 (&sv)[P], float2& nyq) const {
+        if (a.layout == STX_SPEC_F_MAJOR) {
+            const float2* col = sc + frame(s0 + tr % JOBS);
+#pragma unroll
+            for (int i = 0; i < P; i++) sv[i] = col[(size_t)(tr / JOBS + i * TPJ) * a.T];
+            nyq = sc[(size_t)min(M, a.F - 1) * a.T + frame(s0 + min(tr, JOBS - 1))];
+        } else {
+            const float2* row = sc + (size_t)frame(s0 + tr / TPJ) * a.F;
+#pragma unroll
+            for (int i = 0; i < P; i++) sv[i] = row[jr + i * TPJ];
+            nyq = row[min(M, a.F - 1)];
+        }
+    }
+    __device__ __forceinline__ void stage(int tr, int jr, const float2 (&sv)[P], float2 nyq) const {
+        if (a.layout == STX_SPEC_F_MAJOR) {
+            const int g = tr % JOBS, k0 = tr / JOBS;
+#pragma unroll
+            for (int i = 0; i < P; i++) lds[g * SLOT + k0 + i * TPJ] = sv[i];
+            if (tr < JOBS) lds[tr * SLOT + M] = M < a.F ? nyq : make_float2(0.f, 0.f);
+        } else {
+            float2* bs = lds + (tr / TPJ) * SLOT;
+#pragma unroll
+            for (int i = 0; i < P; i++) bs[jr + i * TPJ] = sv[i];
+            if (jr == 0) bs[M] = M < a.F ? nyq : make_float2(0.f, 0.f);
+        }
+    }
+};
+
+// The inverse split and transform of the staged frame in buf, handed to LDS through post (windowed, sample
+// pairs unpadded).
+template <int N, int P, bool WAVE, class Post>
+__device__ __forceinline__ void inverse_frame(float2* buf, int jr, const float2* twt, int keep_nyquist, const Post& post) {
+    constexpr int M = N / 2, TPJ = M / P;
+    // Split twiddles W_N^k for k = jr + r*TPJ: W_N^jr from the table times the constant
+    // W_N^(r*TPJ) = exp(-i pi r / P).
+    constexpr HalfTurnRoots<P> rot = half_turn_roots<P>();
+    const float2 w0 = tw_lookup<N>(twt, jr);
+    float2 v[P];
+#pragma unroll
+    for (int r = 0; r < P; r++) {
+        const int k = jr + r * TPJ;
+        const float2 wr = r == 0 ? w0 : cmul(w0, make_float2(rot.re[r], rot.im[r]));
+        v[r] = inverse_split_w(buf[k], buf[M - k], k, keep_nyquist, wr);
+    }
+    pass_sync<WAVE>();                                  // staging read before the FFT overwrites it
+    fft_first_pass<M, P, N>(v, buf, jr, post, ToLdsFlat{buf});
+    pass_sync<WAVE>();
+    fft_rest_passes<M, P, N, P, WAVE>(buf, jr, twt, post, ToLdsFlat{buf});
+}
+
+// sum * (norm / envelope) where a sample's envelope is summed here (the signal's ends): the window
+// squared of envelope frames tf0 .. tf0 + K in frame order, frame tf0 at position s_first.
+__device__ __forceinline__ float env_quotient(const IstftArgs& a, const float* win, float sum, int tf0, int s_first, int K) {
+    const int i0 = max(0, -tf0), i1 = min(K, a.env_frames - 1 - tf0);
+    unsigned pos = (unsigned)(s_first - i0 * a.hop);
+    float env = 0.f;
+    for (int i = i0; i <= i1; i++, pos -= (unsigned)a.hop) {
+        const float w = win[pos];
+        env += w * w;
+    }
+    return env > 1e-11f ? sum * (a.norm / env) : 0.f;   // as the table's product
+}
+
 // Fused path: one workgroup owns a tile of output samples and inverse-transforms, JOBS frames
 // at a time (normally all at once), every frame that overlaps it; the last FFT pass applies
 // window * norm; each thread sums its samples over the overlapping frames in frame order and
-// divides by the window-squared envelope. PERSIST: fewer workgroups than tiles, each taking
-// several (launches whose tiles outnumber the workgroups the device holds at once).
-template <int N, int P, int JOBS, int PER, bool PERSIST>
+// divides by the window-squared envelope. For calls whose tiles fit on the device at once (more:
+// istft_run_kernel).
+template <int N, int P, int JOBS, int PER>
 __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_kernel(IstftArgs a) {
     constexpr int M = N / 2;
     using C = FftCfg<M, P, N>;
     constexpr int TPJ = C::TPJ;
     constexpr int NT = JOBS * TPJ;
-    // Slots KPW float2 apart modulo 32 (256 bytes of banks): the f-major staging's lanes write
-    // bin tr / JOBS of slot tr % JOBS, KPW = ceil(64 / JOBS) bins per wave, so the JOBS slots'
-    // runs fall on different banks (with slots a multiple of 32 float2 apart they shared them:
-    // 5x the LDS bank-conflict cycles of the t-major staging at c1).
-    constexpr int KPW = (64 + JOBS - 1) / JOBS;                  // a wave is 64 lanes
-    constexpr int SLOT = C::PADN < 512 ? C::PADN : C::PADN + ((KPW - C::PADN % 32) % 32 + 32) % 32;  // short slots: as is
+    constexpr int SLOT = istft_slot<N, P, JOBS>();
     // One wave per transform: between the split and the last pass every lane touches only its
     // own wave's slot, so those passes need no workgroup barrier.
     constexpr bool WAVE = TPJ == 64;
@@ -371,9 +452,8 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_kernel(IstftArgs a) 
     __shared__ float wl[WIN_LDS ? N : 2];
     __shared__ float inv_env[ENV_LDS ? N : 2];
 
-    // Workgroup lb takes tile lb of the a.nblocks tiles over all channels, and with PERSIST also
-    // tiles lb + G, lb + 2G, ... (G = a.grid, the workgroups launched); at every step each XCD
-    // holds a contiguous run of tiles.
+    // Workgroup lb takes tile lb of the a.nblocks tiles over all channels; each XCD holds a
+    // contiguous run of tiles.
     const int lb = xcd_block();
     if (lb >= a.nblocks) return;
     const int tid = (int)threadIdx.x;
@@ -391,55 +471,14 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_kernel(IstftArgs a) 
     const float* win = WIN_LDS ? wl : a.win;
     const WindowMul post{reinterpret_cast<const float2*>(win)};
 
-    struct Tile {
-        int c, J0, J1, st_lo, st_hi;
-        const float2* sc;
-    };
-    auto tile_at = [&](int ti) {
-        Tile t;
-        t.c = ti / a.tiles;
-        const int tile = ti - t.c * a.tiles;
-        t.J0 = max(a.out_off, a.tile_origin + tile * a.tile_len);
-        t.J1 = min(a.out_off + a.out_len, a.tile_origin + (tile + 1) * a.tile_len);
-        // Spectrum frames overlapping [J0, J1): envelope frame tf covers [tf*hop, tf*hop + N).
-        t.st_lo = max(0, max(0, ceildiv(t.J0 - N + 1, hop)) - a.frame_off);
-        t.st_hi = min(a.T - 1, floordiv(t.J1 - 1, hop) - a.frame_off);
-        t.sc = a.spec + (size_t)t.c * a.T * a.F;
-        return t;
-    };
-    // X[0..M] of frames s0 .. s0 + JOBS - 1 into registers, neighbouring lanes on neighbouring
-    // addresses in either layout: bins k < M are P per thread (M * JOBS = P * NT), the Nyquist
-    // bins one per slot; frames past st_hi read frame st_hi again (finite values, transformed
-    // but never summed: the walk stops at st_hi). F-major: element e = tr + i*NT is slot
-    // e % JOBS = tr % JOBS, bin tr / JOBS + i*TPJ. T-major: thread jr of a slot takes bins
-    // jr + i*TPJ of the slot's frame, the FFT's own element order (one row address, then
-    // constant offsets), and the Nyquist bin.
-    auto load_frames = [&](const Tile& t, int s0, int tr, int jr, float2 (&sv)[P], float2& nyq) {
-        if (a.layout == STX_SPEC_F_MAJOR) {
-            const float2* col = t.sc + min(s0 + tr % JOBS, t.st_hi);
-#pragma unroll
-            for (int i = 0; i < P; i++) sv[i] = col[(size_t)(tr / JOBS + i * TPJ) * a.T];
-            nyq = t.sc[(size_t)min(M, a.F - 1) * a.T + min(s0 + min(tr, JOBS - 1), t.st_hi)];
-        } else {
-            const float2* row = t.sc + (size_t)min(s0 + tr / TPJ, t.st_hi) * a.F;
-#pragma unroll
-            for (int i = 0; i < P; i++) sv[i] = row[jr + i * TPJ];
-            nyq = row[min(M, a.F - 1)];
-        }
-    };
-    auto stage_frames = [&](int tr, int jr, const float2 (&sv)[P], float2 nyq) {
-        if (a.layout == STX_SPEC_F_MAJOR) {
-            const int g = tr % JOBS, k0 = tr / JOBS;
-#pragma unroll
-            for (int i = 0; i < P; i++) lds[g * SLOT + k0 + i * TPJ] = sv[i];
-            if (tr < JOBS) lds[tr * SLOT + M] = M < a.F ? nyq : make_float2(0.f, 0.f);
-        } else {
-            float2* bs = lds + (tr / TPJ) * SLOT;
-#pragma unroll
-            for (int i = 0; i < P; i++) bs[jr + i * TPJ] = sv[i];
-            if (jr == 0) bs[M] = M < a.F ? nyq : make_float2(0.f, 0.f);
-        }
-    };
+    const int c = lb / a.tiles, tile = lb - c * a.tiles;
+    const int J0 = max(a.out_off, a.tile_origin + tile * a.tile_len);
+    const int J1 = min(a.out_off + a.out_len, a.tile_origin + (tile + 1) * a.tile_len);
+    // Spectrum frames overlapping [J0, J1): envelope frame tf covers [tf*hop, tf*hop + N).
+    const int st_lo = max(0, max(0, ceildiv(J0 - N + 1, hop)) - a.frame_off);
+    const int st_hi = min(a.T - 1, floordiv(J1 - 1, hop) - a.frame_off);
+    const float2* sc = a.spec + (size_t)c * a.T * a.F;
+    const SpecStage<N, P, JOBS, SLOT> io{a, sc, lds, st_hi};
 
     bool staged = false;
     auto stage_tables = [&]() {
@@ -447,13 +486,6 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_kernel(IstftArgs a) 
         if constexpr (WIN_LDS) wins.store(wl, tid);
         staged = true;
     };
-    Tile t = tile_at(lb);
-    float2 sv[P], nyq = make_float2(0.f, 0.f);
-    if constexpr (PERSIST) {
-        if (t.st_lo <= t.st_hi) load_frames(t, t.st_lo, tid, j, sv, nyq);
-        stage_tables();
-    }
-
     // Samples J = J0 + q*NT + tid (q < PER). With J = A*hop + R (0 <= R < hop), the frames
     // covering J are tf = A - K .. A at positions s = R + K*hop .. R, where K = K0 when
     // R <= rK and K0 - 1 otherwise (K0 = (N-1)/hop, rK = N-1 - K0*hop). One division per
@@ -461,7 +493,7 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_kernel(IstftArgs a) 
     // round's transform rather than held in registers across it.
     const int K0 = (N - 1) / hop, rK = N - 1 - K0 * hop;
     const int dA = NT / hop, dR = NT - dA * hop;
-    auto walk = [&](int J0, int lane, auto&& body) {
+    auto walk = [&](int lane, auto&& body) {
         int A = (J0 + lane) / hop, R = J0 + lane - A * hop;
 #pragma unroll
         for (int q = 0; q < PER; q++) {
@@ -493,108 +525,190 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_kernel(IstftArgs a) 
             inv_env[R] = env > 1e-11f ? a.norm / env : 0.f;
         }
     };
-    if constexpr (ENV_LDS && PERSIST) {
-        lds_barrier();                                // the window table written
-        build_env();                                  // read after the first tile's rounds
-    }
     const float* ldsf = reinterpret_cast<const float*>(lds);
 
-    for (int ti = lb;; ti += a.grid) {
-        const int tn = ti + a.grid;                     // this workgroup's next tile
-        float acc[PER];
+    float acc[PER];
 #pragma unroll
-        for (int q = 0; q < PER; q++) acc[q] = 0.f;
-        for (int s0 = t.st_lo; s0 <= t.st_hi; s0 += JOBS) {
-            // An opaque copy of the lane index: keeps the compiler from hoisting the (round
-            // invariant) twiddle reads, staging addresses and sample walk out of this loop,
-            // which would hold them in registers across the transform.
-            int jr = j, tr = tid;
-            asm volatile("" : "+v"(jr), "+v"(tr));
-            __builtin_assume(jr >= 0 && jr < TPJ && tr >= 0 && tr < NT);
-            if constexpr (PERSIST) {
-                stage_frames(tr, jr, sv, nyq);
-                // The next round's loads (or the next tile's first), in flight through this round.
-                if (s0 + JOBS <= t.st_hi) {
-                    load_frames(t, s0 + JOBS, tr, jr, sv, nyq);
-                } else if (tn < a.nblocks) {
-                    const Tile u = tile_at(tn);
-                    if (u.st_lo <= u.st_hi) load_frames(u, u.st_lo, tr, jr, sv, nyq);
-                }
-            } else {
-                // One tile: each round's frames are loaded at its start, so that no registers are
-                // held across the transform; the tables go to LDS while the first round's loads
-                // are in flight.
-                load_frames(t, s0, tr, jr, sv, nyq);
-                if (!staged) stage_tables();
-                stage_frames(tr, jr, sv, nyq);
-            }
-            lds_barrier();
-            // Split twiddles W_N^k for k = jr + r*TPJ: W_N^jr from the table times the
-            // constant W_N^(r*TPJ) = exp(-i pi r / P).
-            constexpr HalfTurnRoots<P> rot = half_turn_roots<P>();
-            const float2 w0 = tw_lookup<N>(twt, jr);
-            float2 v[P];
-#pragma unroll
-            for (int r = 0; r < P; r++) {
-                const int k = jr + r * TPJ;
-                const float2 wr = r == 0 ? w0 : cmul(w0, make_float2(rot.re[r], rot.im[r]));
-                v[r] = inverse_split_w(buf[k], buf[M - k], k, a.keep_nyquist, wr);
-            }
-            pass_sync<WAVE>();                          // staging read before the FFT overwrites it
-            fft_first_pass<M, P, N>(v, buf, jr, post, ToLdsFlat{buf});
-            pass_sync<WAVE>();
-            fft_rest_passes<M, P, N, P, WAVE>(buf, jr, twt, post, ToLdsFlat{buf});
-            if constexpr (WAVE) lds_barrier();          // every slot written before the sums read them
-            // Slot g now holds samples (2n, 2n + 1) of frame s0 + g at LDS index n (unpadded:
-            // the last pass's lanes write consecutive n), windowed: add the frames of this
-            // round that cover each sample, in frame order.
-            const int s_end = min(t.st_hi, s0 + JOBS - 1);
-            walk(t.J0, tr, [&](int q, int tf0, int s_first, int K) {
-                if (q * NT + tr >= t.J1 - t.J0) return;
-                const int first = tf0 - a.frame_off;              // spectrum frame of tf0
-                const int i0 = max(0, s0 - first), i1 = min(K, s_end - first);
-                // Sample pos (0 <= pos < N) of slot g is float pos of the slot.
-                const float* sl = ldsf + 2 * SLOT * (first + i0 - s0) + (s_first - i0 * hop);
-                float sum = acc[q];
-                for (int i = i0; i <= i1; i++, sl += 2 * SLOT - hop) sum += *sl;
-                acc[q] = sum;
-            });
-            lds_barrier();
-        }
-        if constexpr (PERSIST) {
-            if (t.st_lo > t.st_hi) lds_barrier();      // no frame overlaps the tile (uniform): tables
-        } else {
-            if (!staged) {                             // no frame overlaps the tile (uniform)
-                stage_tables();
-                lds_barrier();
-            }
-            if constexpr (ENV_LDS) {
-                build_env();
-                lds_barrier();
-            }
-        }
-        float* oc = a.out + (size_t)t.c * a.out_len;
-        walk(t.J0, tid, [&](int q, int tf0, int s_first, int K) {
-            const int J = t.J0 + q * NT + tid;
-            if (J >= t.J1) return;
-            float y = 0.f;
-            if (ENV_LDS && J < a.valid_end && tf0 >= 0 && tf0 + K < a.env_frames) {
-                const float r = inv_env[s_first - K * hop];
-                y = r > 0.f ? acc[q] * r : 0.f;
-            } else if (J < a.valid_end) {
-                const int i0 = max(0, -tf0), i1 = min(K, a.env_frames - 1 - tf0);
-                unsigned pos = (unsigned)(s_first - i0 * hop);
-                float env = 0.f;
-                for (int i = i0; i <= i1; i++, pos -= (unsigned)hop) {
-                    const float w = win[pos];
-                    env += w * w;
-                }
-                y = env > 1e-11f ? acc[q] * (a.norm / env) : 0.f;   // as the table's product
-            }
-            store_stream(oc + (J - a.out_off), y);
+    for (int q = 0; q < PER; q++) acc[q] = 0.f;
+    for (int s0 = st_lo; s0 <= st_hi; s0 += JOBS) {
+        // An opaque copy of the lane index: keeps the compiler from hoisting the (round
+        // invariant) twiddle reads, staging addresses and sample walk out of this loop,
+        // which would hold them in registers across the transform.
+        int jr = j, tr = tid;
+        asm volatile("" : "+v"(jr), "+v"(tr));
+        __builtin_assume(jr >= 0 && jr < TPJ && tr >= 0 && tr < NT);
+        // Each round's frames are loaded at its start, so that no registers are held across the
+        // transform; the tables go to LDS while the first round's loads are in flight.
+        float2 sv[P], nyq;
+        io.load(s0, tr, jr, sv, nyq);
+        if (!staged) stage_tables();
+        io.stage(tr, jr, sv, nyq);
+        lds_barrier();
+        inverse_frame<N, P, WAVE>(buf, jr, twt, a.keep_nyquist, post);
+        if constexpr (WAVE) lds_barrier();              // every slot written before the sums read them
+        // Slot g now holds samples (2n, 2n + 1) of frame s0 + g at LDS index n (unpadded:
+        // the last pass's lanes write consecutive n), windowed: add the frames of this
+        // round that cover each sample, in frame order.
+        const int s_end = min(st_hi, s0 + JOBS - 1);
+        walk(tr, [&](int q, int tf0, int s_first, int K) {
+            if (q * NT + tr >= J1 - J0) return;
+            const int first = tf0 - a.frame_off;              // spectrum frame of tf0
+            const int i0 = max(0, s0 - first), i1 = min(K, s_end - first);
+            // Sample pos (0 <= pos < N) of slot g is float pos of the slot.
+            const float* sl = ldsf + 2 * SLOT * (first + i0 - s0) + (s_first - i0 * hop);
+            float sum = acc[q];
+            for (int i = i0; i <= i1; i++, sl += 2 * SLOT - hop) sum += *sl;
+            acc[q] = sum;
         });
-        if (!PERSIST || tn >= a.nblocks) break;
-        t = tile_at(tn);
+        lds_barrier();
+    }
+    if (!staged) {                                     // no frame overlaps the tile (uniform)
+        stage_tables();
+        lds_barrier();
+    }
+    if constexpr (ENV_LDS) {
+        build_env();
+        lds_barrier();
+    }
+    float* oc = a.out + (size_t)c * a.out_len;
+    walk(tid, [&](int q, int tf0, int s_first, int K) {
+        const int J = J0 + q * NT + tid;
+        if (J >= J1) return;
+        float y = 0.f;
+        if (ENV_LDS && J < a.valid_end && tf0 >= 0 && tf0 + K < a.env_frames) {
+            const float r = inv_env[s_first - K * hop];
+            y = r > 0.f ? acc[q] * r : 0.f;
+        } else if (J < a.valid_end) {
+            y = env_quotient(a, win, acc[q], tf0, s_first, K);
+        }
+        store_stream(oc + (J - a.out_off), y);
+    });
+}
+
+// Calls with more tiles than workgroups the device holds: a workgroup takes a run of a.tile_len / hop
+// hops of one channel, round after round of JOBS frames, each frame transformed once (and K0 = (N - 1) /
+// hop frames before the run, whose ends reach into it). A round finishes the samples that end before
+// its last frame does; the sums of its frames over the N - hop samples past them stay in LDS (carry) as
+// the next round's start, so every sample is summed in frame order from +0.0, the tiles' bits. The next
+// round's spectrum loads are in flight through a round's transform (its barriers wait for LDS only).
+// Tiles of JOBS frames transformed ceil(N / hop) - 1 of them twice: at n_fft 4096, hop 1024 8 frames gave
+// 5 hops, at 2048, 441 16 gave 12. T-major, 8 channels of an HTDemucs segment 49.4 -> 31.5 us, 32 RoFormer
+// channels 138 -> 109, 192 727 -> 565 (2.7 TB/s); n_fft 8192, hop 1024 250 -> 90. What is left per round of 16
+// frames at 2048 (16 us) is 10 us of VALU issue and the LDS round trips of passes whose waves move together;
+// two workgroups of 7 frames a CU measured slower (109 -> 152: 130 registers, 14 waves).
+template <int N, int P, int JOBS>
+__global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_run_kernel(IstftArgs a) {
+    constexpr int M = N / 2;
+    using C = FftCfg<M, P, N>;
+    constexpr int TPJ = C::TPJ;
+    constexpr int NT = JOBS * TPJ;
+    constexpr int SLOT = istft_slot<N, P, JOBS>();
+    constexpr bool WAVE = TPJ <= 64;                   // a transform's lanes lie in one wave
+    constexpr int CPER = (N + NT - 1) / NT;            // carry samples per thread
+    __shared__ float2 lds[JOBS * SLOT];
+    __shared__ float2 twt[TwTable<N>::SIZE];
+    __shared__ float wl[N];
+    // [0, min(hop, N)): reciprocal envelope per position R = J mod hop where every covering frame
+    // exists; then the carry (N - hop samples; none for hop >= N).
+    __shared__ float tail[N];
+    const int lb = xcd_block();
+    if (lb >= a.nblocks) return;
+    const int tid = (int)threadIdx.x;
+    const int slot = tid / TPJ;
+    const int j = tid % TPJ;
+    float2* buf = lds + slot * SLOT;
+    const int hop = a.hop;
+    const int c = lb / a.tiles, run = lb - c * a.tiles;
+    const int J0 = max(a.out_off, a.tile_origin + run * a.tile_len);
+    const int J1 = min(a.out_off + a.out_len, a.tile_origin + (run + 1) * a.tile_len);
+    const int K0 = (N - 1) / hop, rK = N - 1 - K0 * hop;
+    const int clen = max(N - hop, 0);
+    float* inv_env = tail;
+    float* carry = tail + min(hop, N);
+    // Envelope frames F0 .. F1 reach into [J0, J1).
+    const int F0 = J0 / hop - K0, F1 = (J1 - 1) / hop;
+    const SpecStage<N, P, JOBS, SLOT> io{a, a.spec + (size_t)c * a.T * a.F, lds, a.T - 1};
+
+    StagedTwiddles<N, NT> tws;
+    Staged<N, NT, float> wins;
+    tws.load(a.twt, tid);
+    wins.load(a.win, tid);
+    float2 sv[P], nyq;
+    io.load(F0 - a.frame_off, tid, j, sv, nyq);
+    tws.store(twt, tid);
+    wins.store(wl, tid);
+    lds_barrier();
+    const WindowMul post{reinterpret_cast<const float2*>(wl)};
+    for (int R = tid; R < min(hop, N); R += NT) {      // read after the first round's barriers
+        float env = 0.f;
+        for (int i = R <= rK ? K0 : K0 - 1; i >= 0; i--) {
+            const float w = wl[R + i * hop];
+            env += w * w;
+        }
+        inv_env[R] = env > 1e-11f ? a.norm / env : 0.f;
+    }
+    const float* ldsf = reinterpret_cast<const float*>(lds);
+    float* oc = a.out + (size_t)c * a.out_len;
+    const int done = JOBS * hop;                       // samples a round finishes, from its first frame's start
+    const int dA = NT / hop, dR = NT - dA * hop;
+    for (int F = F0; F <= F1; F += JOBS) {
+        // Opaque copies, as in istft_kernel.
+        int jr = j, tr = tid;
+        asm volatile("" : "+v"(jr), "+v"(tr));
+        __builtin_assume(jr >= 0 && jr < TPJ && tr >= 0 && tr < NT);
+        io.stage(tr, jr, sv, nyq);
+        if (F + JOBS <= F1) io.load(F + JOBS - a.frame_off, tr, jr, sv, nyq);
+        lds_barrier();
+        inverse_frame<N, P, WAVE>(buf, jr, twt, a.keep_nyquist, post);
+        if constexpr (WAVE) lds_barrier();
+        // Slots of this round that hold spectrum frames.
+        const int s_lo = max(0, a.frame_off - F), s_hi = min(JOBS - 1, a.frame_off + a.T - 1 - F);
+        // Sample x of the round (J = F hop + x) with x = A hop + R: frames A - K .. A of the round.
+        auto frames_at = [&](int x, int A, int R, float sum) {
+            const int K = R <= rK ? K0 : K0 - 1;
+            const int i0 = max(A - K, s_lo), i1 = min(A, s_hi);
+            const float* sl = ldsf + 2 * SLOT * i0 + (x - i0 * hop);
+            for (int i = i0; i <= i1; i++, sl += 2 * SLOT - hop) sum += *sl;
+            return sum;
+        };
+        {
+            int A = tr / hop, R = tr - A * hop;
+            for (int x = tr; x < done; x += NT) {
+                const int J = F * hop + x;
+                if (J >= J0 && J < J1) {
+                    const float sum = frames_at(x, A, R, F > F0 && x < clen ? carry[x] : 0.f);
+                    const int K = R <= rK ? K0 : K0 - 1, tf0 = F + A - K;
+                    float y = 0.f;
+                    if (J < a.valid_end && tf0 >= 0 && tf0 + K < a.env_frames) {
+                        const float r = inv_env[R];
+                        y = r > 0.f ? sum * r : 0.f;
+                    } else if (J < a.valid_end) {
+                        y = env_quotient(a, wl, sum, tf0, R + K * hop, K);
+                    }
+                    store_stream(oc + (J - a.out_off), y);
+                }
+                R += dR;
+                A += dA;
+                if (R >= hop) { R -= hop; A++; }
+            }
+        }
+        if (F + JOBS > F1) break;                      // uniform
+        float cacc[CPER];
+        {
+            int A = (done + tr) / hop, R = done + tr - A * hop;
+#pragma unroll
+            for (int q = 0; q < CPER; q++) {
+                const int x = done + q * NT + tr;
+                cacc[q] = x - done < clen ? frames_at(x, A, R, F > F0 && x < clen ? carry[x] : 0.f) : 0.f;
+                R += dR;
+                A += dA;
+                if (R >= hop) { R -= hop; A++; }
+            }
+        }
+        lds_barrier();                                 // the slots and the old carry read
+#pragma unroll
+        for (int q = 0; q < CPER; q++)
+            if (q * NT + tr < clen) carry[q * NT + tr] = cacc[q];
     }
 }
 
@@ -1134,26 +1248,63 @@ long long plan_istft_tiles(IstftArgs& a, int channels) {
     return (long long)a.tiles * channels;
 }
 
-// One workgroup per tile while the device holds them all at once; past that (MAY_PERSIST), as
-// many workgroups as it holds, each taking every grid-th tile.
-template <int N, int JOBS, bool MAY_PERSIST>
+template <int N, int JOBS>
 void launch_istft_fused_jobs(IstftArgs a, int channels, hipStream_t s) {
     constexpr int P = fused_p(N);
-    constexpr int NT = JOBS * (N / 2 / P);
     a.nblocks = (int)plan_istft_tiles<N, JOBS>(a, channels);
-    if constexpr (MAY_PERSIST) {
-        const void* k = reinterpret_cast<const void*>(istft_kernel<N, P, JOBS, kIstftPer, true>);
-        const int resident = device_blocks(k, NT);
-        if (resident > 0 && a.nblocks > resident) {
-            a.grid = (int)xcd_grid(resident);
-            hipLaunchKernelGGL((istft_kernel<N, P, JOBS, kIstftPer, true>), dim3(a.grid), dim3(NT), 0, s, a);
-            launch_check("istft_kernel");
-            return;
-        }
-    }
-    a.grid = (int)xcd_grid(a.nblocks);
-    hipLaunchKernelGGL((istft_kernel<N, P, JOBS, kIstftPer, false>), dim3(a.grid), dim3(NT), 0, s, a);
+    hipLaunchKernelGGL((istft_kernel<N, P, JOBS, kIstftPer>), dim3(xcd_grid(a.nblocks)), dim3(JOBS * (N / 2 / P)), 0, s, a);
     launch_check("istft_kernel");
+}
+
+// Tiles of istft_kernel that the device holds at once.
+template <int N, int JOBS>
+long long istft_resident() {
+    constexpr int P = fused_p(N);
+    return device_blocks(reinterpret_cast<const void*>(istft_kernel<N, P, JOBS, kIstftPer>), JOBS * (N / 2 / P));
+}
+
+// Frames per workgroup of istft_run_kernel: as many whole waves of them as fit 1,024 threads and the
+// LDS beside the window and the envelope and carry (N floats each). Short frames take 512 threads, two
+// workgroups a CU (n_fft 512, hop 256, 7,814 frames: 16.4 -> 11.8 us, f-major 22.5 -> 15.0; at 1024 it is
+// slower, 67 -> 86).
+constexpr int istft_run_threads(int n) { return n <= 512 ? 512 : 1024; }
+template <int N, int JOBS = block_jobs(N / 2 / fused_p(N), istft_run_threads(N))>
+constexpr int istft_run_jobs() {
+    constexpr int P = fused_p(N), tpj = N / 2 / P;
+    if constexpr (JOBS > 1 && ((size_t)JOBS * istft_slot<N, P, JOBS>() * 8 + TwTable<N>::SIZE * 8 + 2 * (size_t)N * 4 > 160 * 1024 ||
+                               JOBS * tpj % 64 != 0))
+        return istft_run_jobs<N, JOBS - 1>();
+    else
+        return JOBS;
+}
+
+// Runs for calls with more tiles than the device holds workgroups: R rounds of JOBS frames give R JOBS -
+// K0 hops. R is the one whose workgroups (one or two a CU) take the fewest rounds in all, a workgroup's tables
+// and first loads counted as half a round.
+template <int N>
+void launch_istft_runs(IstftArgs a, int channels, hipStream_t s) {
+    constexpr int P = fused_p(N), JOBS = istft_run_jobs<N>();
+    const long long K0 = (N - 1) / a.hop, cus = (long long)device_cus() * (1024 / istft_run_threads(N));
+    const int A0 = a.out_off / a.hop;
+    const long long hops = (a.out_off + (long long)a.out_len - 1) / a.hop - A0 + 1;
+    long long best = 0, best_hops = 1;
+    for (long long R = 1; R <= (hops + K0 + JOBS - 1) / JOBS; R++) {
+        const long long h = R * JOBS - K0;
+        if (h < 1) continue;
+        const long long runs = (hops + h - 1) / h * channels;
+        const long long cost = (runs + cus - 1) / cus * (2 * R + 1);
+        if (best == 0 || cost < best) {
+            best = cost;
+            best_hops = h;
+        }
+        if (runs <= cus) break;                        // longer runs only leave more CUs idle
+    }
+    a.tile_len = (int)std::min<long long>(best_hops, hops) * a.hop;
+    a.tile_origin = A0 * a.hop;
+    a.tiles = (int)((hops + best_hops - 1) / best_hops);
+    a.nblocks = a.tiles * channels;
+    hipLaunchKernelGGL((istft_run_kernel<N, P, JOBS>), dim3(xcd_grid(a.nblocks)), dim3(JOBS * (N / 2 / P)), 0, s, a);
+    launch_check("istft_run_kernel");
 }
 
 // One workgroup per CU at most (the frames fill the LDS), so when the full-size tiles leave
@@ -1169,11 +1320,13 @@ void launch_istft_fused(IstftArgs a, int channels, hipStream_t s) {
         const long long cus = device_cus();
         if (ALT - span >= 1 && plan_istft_tiles<N, JOBS>(t, channels) < cus &&
             plan_istft_tiles<N, ALT>(t, channels) <= cus) {
-            launch_istft_fused_jobs<N, ALT, false>(a, channels, s);
+            launch_istft_fused_jobs<N, ALT>(a, channels, s);
             return;
         }
     }
-    launch_istft_fused_jobs<N, JOBS, true>(a, channels, s);
+    IstftArgs t = a;
+    if (plan_istft_tiles<N, JOBS>(t, channels) > istft_resident<N, JOBS>()) launch_istft_runs<N>(a, channels, s);
+    else launch_istft_fused_jobs<N, JOBS>(a, channels, s);
 }
 
 // The several-frames kernels' workgroups: 16 frames of frame_threads() threads. 0: not for this plan or

@@ -238,8 +238,8 @@ def test_small_hop_needs_several_rounds(device, orc):
     (1024, 8, 2000, 8, 1),          # 4 rounds of 32 frames per tile: 2,000 tiles; 1 channel: 250
 ])
 def test_istft_more_tiles_than_resident_workgroups(device, orc, layout, n, hop, length, channels, sub):
-    # A batch whose tiles outnumber the workgroups the GPU holds at once: each workgroup takes
-    # several tiles (and prefetches the next tile's frames). Every channel must equal, bit for
+    # A batch whose tiles outnumber the workgroups the GPU holds at once: each workgroup takes a
+    # run of hops (and prefetches the next round's frames). Every channel must equal, bit for
     # bit, the same channels inverted in a call small enough to give each tile its own workgroup.
     x = synth.normal(4100 + n, (channels, length), 0.2)
     f = plan(n)
@@ -258,8 +258,8 @@ def test_istft_more_tiles_than_resident_workgroups(device, orc, layout, n, hop, 
 
 @pytest.mark.parametrize("layout", [stx.F_MAJOR, stx.T_MAJOR])
 def test_htdemucs_ispec_many_segments_same_bits_as_pairs(device, orc, layout):
-    # 16 HTDemucs segments (n_fft 4096) in one call: 8-frame tiles of 5 hops, 1,088 of them,
-    # several per workgroup; a call of two segments takes 6-frame tiles of 3 hops, one per
+    # 16 HTDemucs segments (n_fft 4096) in one call: 1,088 tiles of 5 hops, so runs of rounds of 7
+    # frames; a call of two segments takes 6-frame tiles of 3 hops, one per
     # workgroup. Each sample adds the same frames in the same order either way, so every
     # channel must come out bit for bit the same.
     length, channels = 343980, 16
@@ -276,6 +276,34 @@ def test_htdemucs_ispec_many_segments_same_bits_as_pairs(device, orc, layout):
         ref = orc.htdemucs_spec(x[c], 4096)
         assert snr_db(s, ref) >= SNR_DB
         assert snr_db(y[c], orc.htdemucs_ispec(ref, 4096, length)) >= SNR_DB
+
+
+# Runs of istft_run_kernel at its edges: n_fft 8192 (two frames a round, the carry longer than a round finishes), hop n
+# (no carry), hops that leave one sample uncovered (n - 1) or divide nothing, one sample past a run's end, and every
+# power of two from 16 (many frames a round).
+RUN_CASES = [(8192, 1024, 1024 * 400 + 5, 3), (8192, 333, 333 * 500, 2), (4096, 1023, 1023 * 700 + 1, 2), (2048, 2048, 2048 * 500, 9),
+             (2048, 2047, 2047 * 700, 5), (1024, 300, 300 * 9001, 2), (512, 128, 128 * 17000 + 3, 2), (256, 64, 64 * 20001, 2),
+             (128, 50, 50 * 30001, 2), (64, 16, 16 * 70001, 1), (32, 8, 8 * 400001, 1), (16, 4, 4 * 400001, 1)]
+
+
+@pytest.mark.parametrize("layout", [stx.F_MAJOR, stx.T_MAJOR])
+@pytest.mark.parametrize("n,hop,length,channels", RUN_CASES)
+def test_istft_runs(device, orc, layout, n, hop, length, channels):
+    """Calls with more tiles than the device holds workgroups against the oracle's inverse of the same spectrum (every
+    channel equal, so that one oracle run serves; channels of a call are independent runs)."""
+    x = synth.normal(4400 + n + hop, (1, length), 0.2)
+    f = plan(n)
+    one = stx.torch_stft(f, to_dev(x, device), hop, layout=layout)
+    spec = one.expand(channels, -1, -1).contiguous()
+    y = host(stx.torch_istft(f, spec, hop, layout=layout))
+    s = host(one)[0]
+    ref = orc.torch_istft((s if layout == stx.F_MAJOR else s.T).astype(np.complex128), n, hop)
+    w = 0.5 - 0.5 * np.cos(2.0 * np.pi * np.arange(n) / n)
+    env = np.array([np.sum(w[r::hop] ** 2) for r in range(hop)])
+    loss = max(0.0, 10.0 * np.log10(np.mean(1.0 / env[env > 1e-11])))   # a sample's error: the frames' over sqrt(env)
+    assert snr_db(y[0], ref) >= SNR_DB - loss
+    for c in range(1, channels):
+        assert np.array_equal(y[c], y[0])
 
 
 def test_istft_many_tiles_graph_replays(device):
