@@ -207,27 +207,17 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void stft_kernel(StftArgs a) {
             }
         }
     } else {
-        // Row of frame g, then each bin's twiddle once for all JOBS frames.
-        constexpr int KSP = NT + NT / P;
-        float2* rows[JOBS];
+        // The thread's own frame: bins j + i*TPJ, the same twiddles as above.
+        constexpr int KSP = TPJ + TPJ / P;
+        if (active) {
+            float2* row = a.spec + ((size_t)c * a.T + t) * a.F;
+            int ik = C::idx(j), im = C::idx(M - j);
+            const float2 w0 = tw_lookup<N>(twt, j);
 #pragma unroll
-        for (int g = 0; g < JOBS; g++) {
-            int tt = t0 + g, cc = c0;
-            while (tt >= a.T) { tt -= a.T; cc++; }
-            rows[g] = f0 + g < a.jobs ? a.spec + ((size_t)cc * a.T + tt) * a.F : nullptr;
-        }
-        // Bin stride NT = JOBS * TPJ: W_N^(i*NT) = exp(-i pi i JOBS / P).
-        static_assert(P % JOBS == 0, "t-major bin stride");
-        int ik = C::idx(tid), im = C::idx(M - tid);
-        const float2 w0 = tw_lookup<N>(twt, tid);
-#pragma unroll
-        for (int i = 0; i <= P / JOBS; i++, ik += KSP, im -= KSP) {   // tid + (P / JOBS) * NT >= M
-            const int k = tid + i * NT;
-            if (k >= a.F) continue;
-            const float2 w = rotate(w0, i * JOBS);
-#pragma unroll
-            for (int g = 0; g < JOBS; g++)
-                if (rows[g]) store_stream(rows[g] + k, bin(lds + g * SLOT, k, ik, im, w, std::integral_constant<int, NT>{}));
+            for (int i = 0; i <= P; i++, ik += KSP, im -= KSP) {   // j + P*TPJ >= M
+                const int k = j + i * TPJ;
+                if (k < a.F) store_stream(row + k, bin(buf, k, ik, im, rotate(w0, i), std::integral_constant<int, TPJ>{}));
+            }
         }
     }
 }
@@ -1214,8 +1204,6 @@ constexpr int kIstftPer = 6;                           // fused: output samples 
 constexpr int kStftP = 8;
 constexpr int fused_p(int n) { return n / 2 >= 16 ? 16 : 8; }
 
-// One frame per workgroup in the T-major layout (the most workgroups); two in the F-major
-// layout, whose bins then leave as 16-byte runs of two frames per row instead of 8.
 template <int N, int JOBS>
 void launch_stft_jobs(StftArgs a, hipStream_t s) {
     constexpr int P = kStftP;
@@ -1225,12 +1213,27 @@ void launch_stft_jobs(StftArgs a, hipStream_t s) {
     launch_check("stft_kernel");
 }
 
+// Frames per workgroup. Few frames: one in the T-major layout (the most workgroups), two in the
+// F-major layout, whose bins then leave as 16-byte runs of two frames per row instead of 8. From
+// kStftMany frames on, when they fill the device several times over, F-major rows take runs of four
+// frames (32 stereo chunks at n_fft 2048, hop 441: 115 -> 84 us; 8 frames 96), short frames of either
+// layout eight and 1,024-point frames in rows of their own four (n_fft 128, hop 64, 62,502 frames: 29 -> 16 us,
+// T-major 48 -> 23; n_fft 1024: 54 -> 42, 39 -> 36).
+constexpr int kStftMany = 2048;
+
 template <int N>
 void launch_stft(const StftArgs& a, hipStream_t s) {
     constexpr int TPJ = N / 2 / kStftP;
-    constexpr int J2 = TPJ * 2 <= 1024 ? 2 : 1;
-    if (a.layout == STX_SPEC_T_MAJOR) launch_stft_jobs<N, 1>(a, s);
-    else launch_stft_jobs<N, J2>(a, s);
+    constexpr bool SHORT = N <= 512;
+    constexpr int J2 = TPJ * 2 <= 1024 ? 2 : 1, FMANY = SHORT ? 8 : TPJ * 4 <= 1024 ? 4 : J2, TMANY = SHORT ? 8 : N == 1024 ? 4 : 1;
+    const bool many = a.jobs >= kStftMany;
+    if (a.layout == STX_SPEC_T_MAJOR) {
+        if (TMANY > 1 && many) launch_stft_jobs<N, TMANY>(a, s);
+        else launch_stft_jobs<N, 1>(a, s);
+    } else {
+        if (FMANY > J2 && many) launch_stft_jobs<N, FMANY>(a, s);
+        else launch_stft_jobs<N, J2>(a, s);
+    }
 }
 
 // Tiles of m hops need m + ceil(N/hop) - 1 frames; m is chosen so that they fit one round of

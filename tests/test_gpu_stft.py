@@ -278,6 +278,27 @@ def test_htdemucs_ispec_many_segments_same_bits_as_pairs(device, orc, layout):
         assert snr_db(y[c], orc.htdemucs_ispec(ref, 4096, length)) >= SNR_DB
 
 
+# The switch to several frames a workgroup (2,048 frames), the last workgroup partly past the end and workgroups that
+# cross channels, for every group size (8, 4 and 1).
+@pytest.mark.parametrize("layout", [stx.F_MAJOR, stx.T_MAJOR])
+@pytest.mark.parametrize("n,hop,length,channels", [(2048, 441, 441 * 1025, 2), (2048, 441, 441 * 682 + 3, 3), (1024, 256, 256 * 410 + 9, 5),
+                                                   (512, 128, 128 * 1026, 2), (128, 64, 64 * 2049 + 1, 1), (16, 4, 4 * 1030, 2),
+                                                   (8192, 2048, 2048 * 420, 5), (4096, 1024, 1024 * 684, 3)])
+def test_stft_many_frames(device, orc, layout, n, hop, length, channels):
+    """STFT calls of 2,048 frames and more: every channel has the bits of a call of its own (fewer frames, one or two a
+    workgroup), and the oracle's values."""
+    x = synth.normal(4500 + n + hop, (channels, length), 0.2)
+    f, xd = plan(n), to_dev(x, device)
+    assert channels * (length // hop + 1) >= 2048
+    spec = host(stx.torch_stft(f, xd, hop, layout=layout))
+    for c in range(channels):
+        if length // hop + 1 < 2048:
+            one = host(stx.torch_stft(f, xd[c:c + 1].contiguous(), hop, layout=layout))
+            assert np.array_equal(one[0], spec[c])
+        s = spec[c] if layout == stx.F_MAJOR else spec[c].T
+        assert snr_db(s, orc.torch_stft(x[c], n, hop)) >= SNR_DB
+
+
 # Runs of istft_run_kernel at its edges: n_fft 8192 (two frames a round, the carry longer than a round finishes), hop n
 # (no carry), hops that leave one sample uncovered (n - 1) or divide nothing, one sample past a run's end, and every
 # power of two from 16 (many frames a round).
