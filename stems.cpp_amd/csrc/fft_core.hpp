@@ -588,6 +588,9 @@ __device__ __forceinline__ float2* mixed_fft_ct(float2* src, float2* dst, const 
     else return mixed_fft_ct<NT, M, TWMUL, Ns * R, Rest...>(dst, src, twl, tid);
 }
 
+template <int TPF, int M, int TWMUL, int R, int... Rest, class TW>
+__device__ __forceinline__ void frame_passes_after(float2* buf, const TW& tw, int j);
+
 // A transform size whose plan (the radices mixed_plan gives) is compiled in: mixed_fft_ct over
 // M points. The host checks that the plan object it built has the same radices.
 template <int M_, int... Rs>
@@ -598,6 +601,11 @@ struct MixedCt {
     template <int NT, int TWMUL>
     static __device__ __forceinline__ float2* run(float2* b0, float2* b1, const float2* twl, int tid) {
         return mixed_fft_ct<NT, M, TWMUL, 1, Rs...>(b0, b1, twl, tid);
+    }
+    // The passes after the first, in place by TPF threads (frame_pass).
+    template <int TPF, int TWMUL, class TW>
+    static __device__ __forceinline__ void frame_rest(float2* buf, const TW& tw, int j) {
+        frame_passes_after<TPF, M, TWMUL, Rs...>(buf, tw, j);
     }
 };
 // Kim_Vocal_2's n_fft 7680: the real transform's 3840-point half.
@@ -702,6 +710,11 @@ template <int TPF, int M, int TWMUL, int Ns, int R, int... Rest, class TW>
 __device__ __forceinline__ void frame_passes_ct(float2* buf, const TW& tw, int j) {
     frame_pass<R, TPF, M, Ns>(buf, M, Ns, (M / (Ns * R)) * TWMUL, tw, j);
     if constexpr (sizeof...(Rest) > 0) frame_passes_ct<TPF, M, TWMUL, Ns * R, Rest...>(buf, tw, j);
+}
+
+template <int TPF, int M, int TWMUL, int R, int... Rest, class TW>
+__device__ __forceinline__ void frame_passes_after(float2* buf, const TW& tw, int j) {
+    if constexpr (sizeof...(Rest) > 0) frame_passes_ct<TPF, M, TWMUL, R, Rest...>(buf, tw, j);
 }
 
 // The first pass of a plan that starts with radix 16, from registers: v holds elements

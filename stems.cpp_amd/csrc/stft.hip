@@ -723,8 +723,8 @@ __device__ __forceinline__ int padded_index_rt(int m, const StftArgs& a, int n) 
 
 // CT: a size whose plan is compiled in (MixedCt: constant trip counts, LDS offsets as
 // immediates), or void for the plan p at run time.
-template <class CT> struct MixedM { static constexpr int value = CT::M; };
-template <> struct MixedM<void> { static constexpr int value = 0; };
+template <class CT> struct MixedM { static constexpr int value = CT::M, first = CT::radix[0]; };
+template <> struct MixedM<void> { static constexpr int value = 0, first = 0; };
 
 // FPB frames per block, as in istft_frames_mixed_kernel: with FPB = 2 (f-major, T even, 16-byte
 // aligned spectrum) the two frames t and t + 1 of one channel are transformed by the two halves
@@ -895,6 +895,9 @@ __global__ __launch_bounds__(kMixedThreads * FPB) void istft_frames_mixed_kernel
 // passes need no barrier. The twiddles are the full table of W_n^m in LDS for n <= 2048. Bound by LDS
 // traffic and VALU issue: n_fft 960, hop 480, a minute of stereo f-major 120 -> 24.9 us (3.4 TB/s of the
 // signal and the spectrum), iSTFT 143 -> 37.9; n_fft 320, hop 80, 12,502 frames 95 -> 15.3 and 109 -> 19.3.
+// With 128 and 256 threads a frame (n up to 7680 and 8192) the passes have barriers, and what counts is the one LDS
+// buffer a frame: two workgroups of 2 frames a CU, where stft_mixed_kernel's two ping-pong buffers held 2 frames in
+// all. n_fft 7680, 2,048 frames f-major: STFT 53 -> 40 us, iSTFT 71 -> 61; 4 frames a workgroup 42 and 63.
 constexpr int kFrameTw = 2048;                         // full tables up to this n
 
 // Dynamic LDS: JOBS slots of frame_slot(M) float2, then the twiddles, then (iSTFT) the window.
@@ -917,29 +920,53 @@ struct StagedRt {
     }
 };
 
-template <int TPF, int JOBS>
-__global__ __launch_bounds__(TPF * JOBS) __attribute__((amdgpu_waves_per_eu(4))) void stft_frames_kernel(StftArgs a, MixedRadix p, const float2* __restrict__ twn, int n,
-                                                                 FastDiv ft) {
+// The frame's twiddles and transform: v holds its elements j + u step (step = M / 16 for a plan that
+// starts with radix 16, which runs its first pass from the registers, else TPF). Ends with a
+// frame_sync; `publish` runs between the first pass and the next (a barrier that publishes the twiddles).
+template <int TPF, class CT, class TW, class Publish>
+__device__ __forceinline__ void frame_transform(float2 (&v)[16], float2* buf, int M, const MixedRadix& p, const TW& tw, int j,
+                                                Publish&& publish) {
+    const bool first16 = (MixedM<CT>::value ? MixedM<CT>::first : p.r[0]) == 16;
+    if (first16) {
+        frame_first16<TPF>(v, buf, M, j);
+    } else {
+#pragma unroll
+        for (int u = 0; u < 16; u++)
+            if (j + u * TPF < M) buf[mixed_pad(j + u * TPF)] = v[u];
+        frame_sync<TPF>();
+    }
+    publish();
+    if constexpr (MixedM<CT>::value != 0) CT::template frame_rest<TPF, 2>(buf, tw, j);
+    else frame_passes<TPF>(buf, M, p, first16 ? 1 : 0, first16 ? 16 : 1, 2, tw, j);
+}
+template <int TPF, class CT>
+__device__ __forceinline__ int frame_step(int M, const MixedRadix& p) {
+    return (MixedM<CT>::value ? MixedM<CT>::first : p.r[0]) == 16 ? M / 16 : TPF;
+}
+
+template <int TPF, int JOBS, class CT>
+__global__ __launch_bounds__(TPF * JOBS) __attribute__((amdgpu_waves_per_eu(4))) void stft_frames_kernel(
+    StftArgs a, MixedRadix p, const float2* __restrict__ twn, const float2* __restrict__ twm, int n_rt, FastDiv ft) {
     extern __shared__ float2 sm[];
     constexpr int NT = TPF * JOBS;
+    constexpr bool FULL = TPF <= 64;                   // n <= kFrameTw: the full twiddle table in LDS
+    const int n = MixedM<CT>::value ? 2 * MixedM<CT>::value : n_rt;
     const int M = n / 2, slot = frame_slot(M);
     const int lb = xcd_block();
     if (lb >= a.nblocks) return;                       // whole block idle: no barrier reached
     const int tid = (int)threadIdx.x, g = tid / TPF, j = tid % TPF;
     float2* buf = sm + g * slot;
     float2* twl = sm + JOBS * slot;
-    StagedRt<kFrameTw, NT, float2> tws;
-    tws.load(twn, n, tid);
+    StagedRt<FULL ? kFrameTw : kMixedTwMax, NT, float2> tws;
+    const int twc = FULL ? n : kMixedTwMax;
+    tws.load(FULL ? twn : twm, twc, tid);
     const int f0 = lb * JOBS, f = min(f0 + g, a.jobs - 1);      // past the end: the last frame again, not written
     const int c = (int)ft.div((unsigned)f), t = f - c * a.T;
     const float* xc = a.x + (size_t)c * a.len;
     const int m0 = a.frame0 + t * a.hop;
     const int base = m0 - M - a.pre_left;              // its signal index when nothing reflects
     const bool interior = base >= 0 && base + n <= a.len;
-    // Elements j + u step: the first pass's own order when it is a radix-16 one (straight from the
-    // registers), else one after the other.
-    const bool first16 = p.r[0] == 16;
-    const int step = first16 ? M / 16 : TPF;
+    const int step = frame_step<TPF, CT>(M, p);
     const float2* win2 = reinterpret_cast<const float2*>(a.win);
     float2 v[16];
     auto element = [&](int u) { return min(j + u * step, M - 1); };
@@ -962,20 +989,14 @@ __global__ __launch_bounds__(TPF * JOBS) __attribute__((amdgpu_waves_per_eu(4)))
     for (int u = 0; u < 16; u++) w[u] = win2[element(u)];
 #pragma unroll
     for (int u = 0; u < 16; u++) v[u] = make_float2(v[u].x * w[u].x, v[u].y * w[u].y);
-    tws.store(twl, n, tid);
-    if (first16) {
-        frame_first16<TPF>(v, buf, M, j);
-    } else {
-#pragma unroll
-        for (int u = 0; u < 16; u++)
-            if (j + u * TPF < M) buf[mixed_pad(j + u * TPF)] = v[u];
-    }
-    __syncthreads();                                   // the twiddles
-    frame_passes<TPF>(buf, M, p, first16 ? 1 : 0, first16 ? 16 : 1, 2, TwFull{twl}, j);
-    // X[k] = E[k] + W_n^k O[k], k <= n/2, as in stft_kernel.
+    tws.store(twl, twc, tid);
+    using TW = typename std::conditional<FULL, TwFull, TwTwoLevel>::type;
+    frame_transform<TPF, CT>(v, buf, M, p, TW{twl}, j, [] { __syncthreads(); });
+    // X[k] = E[k] + W_n^k O[k], k <= n/2, as in stft_kernel; W_n^k from the full table.
     const float hs = 0.5f * a.scale;
-    auto bin = [&](const float2* z, int k) {
-        const float2 zk = z[mixed_pad(k == M ? 0 : k)], zm = z[mixed_pad(k == 0 ? 0 : M - k)], w = twl[k];
+    const float2* wk = FULL ? twl : twn;
+    auto bin = [&](const float2* z, int k, float2 w) {
+        const float2 zk = z[mixed_pad(k == M ? 0 : k)], zm = z[mixed_pad(k == 0 ? 0 : M - k)];
         const float er = zk.x + zm.x, ei = zk.y - zm.y;
         const float orr = zk.y + zm.y, oi = zm.x - zk.x;
         return make_float2((er + w.x * orr - w.y * oi) * hs, (ei + w.x * oi + w.y * orr) * hs);
@@ -987,11 +1008,37 @@ __global__ __launch_bounds__(TPF * JOBS) __attribute__((amdgpu_waves_per_eu(4)))
         const int cc = (int)ft.div((unsigned)ff), tt = ff - cc * a.T;
         const float2* z = sm + gg * slot;
         float2* col = a.spec + (size_t)cc * a.F * a.T + tt;
-        for (int k = tid / JOBS; k < a.F; k += TPF) col[(size_t)k * a.T] = bin(z, k);
+#pragma unroll 4
+        for (int k = tid / JOBS; k < a.F; k += TPF) col[(size_t)k * a.T] = bin(z, k, wk[k]);
     } else if (f0 + g < a.jobs) {
         float2* row = a.spec + ((size_t)c * a.T + t) * a.F;
-        for (int k = j; k < a.F; k += TPF) store_stream(row + k, bin(buf, k));
+        for (int k = j; k < a.F; k += TPF) store_stream(row + k, bin(buf, k, wk[k]));
     }
+}
+
+// Bins 0..M of spectrum frames s .. s + JOBS - 1 (past `last`: frame `last` again) to their slots, neighbouring
+// lanes on neighbouring addresses in either layout, every load before the first LDS write; `between` runs
+// while they are in flight. The caller's barrier publishes them.
+template <int TPF, int JOBS, class Between>
+__device__ __forceinline__ void frame_bins(const IstftArgs& a, const float2* sc, int s, int last, int M, float2* sm, int slot,
+                                           int tid, Between&& between) {
+    const bool fm = a.layout == STX_SPEC_F_MAJOR;
+    const int g = fm ? tid % JOBS : tid / TPF, k0 = fm ? tid / JOBS : tid % TPF;
+    float2 x[17];
+    if (fm) {
+        const float2* col = sc + min(s + g, last);
+#pragma unroll
+        for (int i = 0; i < 17; i++) x[i] = col[(size_t)min(k0 + i * TPF, min(M, a.F - 1)) * a.T];
+    } else {
+        const float2* row = sc + (size_t)min(s + g, last) * a.F;
+#pragma unroll
+        for (int i = 0; i < 17; i++) x[i] = row[min(k0 + i * TPF, min(M, a.F - 1))];
+    }
+    between();
+    float2* xs = sm + g * slot;
+#pragma unroll
+    for (int i = 0; i < 17; i++)
+        if (k0 + i * TPF <= M) xs[mixed_pad(k0 + i * TPF)] = x[i];
 }
 
 // The iSTFT of the same sizes with the overlap-add in the workgroup, as istft_kernel's: a tile of
@@ -1021,29 +1068,12 @@ __global__ __launch_bounds__(TPF * JOBS) __attribute__((amdgpu_waves_per_eu(4)))
     const int st_hi = min(a.T - 1, floordiv(J1 - 1, a.hop) - a.frame_off);
     const float2* sc = a.spec + (size_t)c * a.T * a.F;
     if (st_lo <= st_hi) {                              // uniform
-        // Bins 0..M of every frame (past st_hi: frame st_hi again, never summed), neighbouring
-        // lanes on neighbouring addresses in either layout, every load before the first LDS write.
-        float2 x[17];
-        if (a.layout == STX_SPEC_F_MAJOR) {
-            const float2* col = sc + min(st_lo + tid % JOBS, st_hi);
-#pragma unroll
-            for (int i = 0; i < 17; i++) x[i] = col[(size_t)min(tid / JOBS + i * TPF, min(M, a.F - 1)) * a.T];
-        } else {
-            const float2* row = sc + (size_t)min(st_lo + g, st_hi) * a.F;
-#pragma unroll
-            for (int i = 0; i < 17; i++) x[i] = row[min(j + i * TPF, min(M, a.F - 1))];
-        }
-        tws.store(twl, n, tid);
-        wins.store(win, n, tid);
-        const bool fm = a.layout == STX_SPEC_F_MAJOR;
-        float2* xs = sm + (fm ? tid % JOBS : g) * slot;
-        const int k0 = fm ? tid / JOBS : j;
-#pragma unroll
-        for (int i = 0; i < 17; i++)
-            if (k0 + i * TPF <= M) xs[mixed_pad(k0 + i * TPF)] = x[i];
+        frame_bins<TPF, JOBS>(a, sc, st_lo, st_hi, M, sm, slot, tid, [&] {
+            tws.store(twl, n, tid);
+            wins.store(win, n, tid);
+        });
         __syncthreads();
-        const bool first16 = p.r[0] == 16;
-        const int step = first16 ? M / 16 : TPF;
+        const int step = frame_step<TPF, void>(M, p);
         float2 v[16];
 #pragma unroll
         for (int u = 0; u < 16; u++) {
@@ -1051,15 +1081,7 @@ __global__ __launch_bounds__(TPF * JOBS) __attribute__((amdgpu_waves_per_eu(4)))
             v[u] = inverse_split_w(buf[mixed_pad(k)], buf[mixed_pad(M - k)], k, a.keep_nyquist, twl[k]);
         }
         frame_sync<TPF>();                             // the bins read before the transform overwrites them
-        if (first16) {
-            frame_first16<TPF>(v, buf, M, j);
-        } else {
-#pragma unroll
-            for (int u = 0; u < 16; u++)
-                if (j + u * TPF < M) buf[mixed_pad(j + u * TPF)] = v[u];
-            frame_sync<TPF>();
-        }
-        frame_passes<TPF>(buf, M, p, first16 ? 1 : 0, first16 ? 16 : 1, 2, TwFull{twl}, j);
+        frame_transform<TPF, void>(v, buf, M, p, TwFull{twl}, j, [] {});
     } else {
         wins.store(win, n, tid);
     }
@@ -1080,6 +1102,60 @@ __global__ __launch_bounds__(TPF * JOBS) __attribute__((amdgpu_waves_per_eu(4)))
             }
         }
         store_stream(oc + (J - a.out_off), J < a.valid_end && env > 1e-11f ? sum / env : 0.f);
+    }
+}
+
+// The iSTFT of larger n with many frames, step 1 (step 2 is istft_ola_kernel): JOBS neighbouring frames a workgroup
+// inverse-transformed and written windowed to the workspace, as istft_frames_mixed_kernel's, in half its LDS.
+template <int TPF, int JOBS, class CT>
+__global__ __launch_bounds__(TPF * JOBS) __attribute__((amdgpu_waves_per_eu(4))) void istft_frames_kernel(
+    IstftArgs a, MixedRadix p, const float2* __restrict__ twn, const float2* __restrict__ twm, int n_rt, int groups, FastDiv fg) {
+    extern __shared__ float2 sm[];
+    constexpr int NT = TPF * JOBS;
+    const int n = MixedM<CT>::value ? 2 * MixedM<CT>::value : n_rt;
+    const int M = n / 2, slot = frame_slot(M);
+    const int lb = xcd_block();
+    if (lb >= a.nblocks) return;                       // whole block idle: no barrier reached
+    const int tid = (int)threadIdx.x, g = tid / TPF, j = tid % TPF;
+    float2* buf = sm + g * slot;
+    float2* twl = sm + JOBS * slot;
+    StagedRt<kMixedTwMax, NT, float2> tws;
+    tws.load(twm, kMixedTwMax, tid);
+    // Groups of frames of one channel: group q holds frames q JOBS ...
+    const int c = (int)fg.div((unsigned)lb), st = (lb - c * groups) * JOBS, last = min(st + JOBS, a.T) - 1;
+    frame_bins<TPF, JOBS>(a, a.spec + (size_t)c * a.T * a.F, st, last, M, sm, slot, tid,
+                          [&] { tws.store(twl, kMixedTwMax, tid); });
+    const int step = frame_step<TPF, CT>(M, p);
+    float2 w[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) w[u] = twn[min(j + u * step, M - 1)];
+    __syncthreads();
+    float2 v[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+        const int k = min(j + u * step, M - 1);
+        v[u] = inverse_split_w(buf[mixed_pad(k)], buf[mixed_pad(M - k)], k, a.keep_nyquist, w[u]);
+    }
+    frame_sync<TPF>();                                 // the bins read before the transform overwrites them
+    frame_transform<TPF, CT>(v, buf, M, p, TwTwoLevel{twl}, j, [] {});
+    if (st + g > last) return;
+    float* dst = a.frames + ((size_t)c * a.T + st + g) * n;
+    const float2* win2 = reinterpret_cast<const float2*>(a.win);
+    const bool pairs = (reinterpret_cast<uintptr_t>(a.frames) & 7) == 0;   // n is even
+#pragma unroll
+    for (int u = 0; u < 16; u++) w[u] = win2[min(j + u * TPF, M - 1)];
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+        const int i = j + u * TPF;
+        if (i >= M) break;
+        const float2 r = buf[mixed_pad(i)];
+        const float2 o = make_float2(r.x * w[u].x * a.norm, -r.y * w[u].y * a.norm);
+        if (pairs) {
+            store_stream(reinterpret_cast<float2*>(dst + 2 * i), o);
+        } else {
+            store_stream(dst + 2 * i, o.x);
+            store_stream(dst + 2 * i + 1, o.y);
+        }
     }
 }
 
@@ -1332,67 +1408,100 @@ void launch_istft_fused(IstftArgs a, int channels, hipStream_t s) {
     else launch_istft_fused_jobs<N, JOBS>(a, channels, s);
 }
 
-// The several-frames kernels' workgroups: 16 frames of frame_threads() threads. 0: not for this plan or
-// this many frames (channels times frames): below about 1,024 they leave CUs idle and one frame a
-// workgroup is faster (n_fft 960, 368 frames: 8.7 against 9.6 us, iSTFT 11.9 against 13.6; 11,026
-// frames: 120 against 24.9, iSTFT 143 against 37.9).
+// The several-frames kernels' workgroups: 16 frames of frame_threads() threads (16, 32 or 64; n <= kFrameTw), 4 of
+// 128 or 2 of 256. 0: not for this plan or this many frames (channels times frames): with few, one frame a
+// workgroup of 512 threads is faster. Up to 64 threads below about 1,024 frames (n_fft 960, 368 frames: 8.7 against
+// 9.6 us, iSTFT 11.9 against 13.6; 11,026 frames: 120 against 23, iSTFT 143 against 35); 128 and 256 up to the two
+// frames a CU that those workgroups hold at once (n_fft 7680 f-major, 512 frames: 16.6 against 16.4 and 23.7 against
+// 24.5 us; 768: 25.5 against 19.7, 35.9 against 28.6).
 constexpr int kFrameJobs = 16;
 constexpr int kFrameMinJobs = 1024;
+template <int TPF> constexpr int frame_jobs() { return TPF <= 64 ? kFrameJobs : TPF == 128 ? 4 : 2; }
 int frames_plan(const stx_fft* f, long long jobs) {
-    if (jobs < kFrameMinJobs) return 0;
-    const int t = f->n <= kFrameTw ? frame_threads(f->n / 2, f->half) : 0;
-    return t <= 64 ? t : 0;
+    const int t = frame_threads(f->n / 2, f->half);
+    return jobs >= (t <= 64 ? kFrameMinJobs : 2LL * device_cus() + 1) ? t : 0;
 }
 
-// Calls go(integral_constant<int, TPF>) for t = 16, 32 or 64.
+// Calls go(integral_constant<int, TPF>, CT*) for t threads a frame, CT the compiled plan of n_fft 7680 or void.
 template <class F>
-void pick_frame_threads(int t, F&& go) {
+void pick_frame_threads(const stx_fft* f, int t, F&& go) {
     using std::integral_constant;
-    if (t == 16) go(integral_constant<int, 16>{});
-    else if (t == 32) go(integral_constant<int, 32>{});
-    else go(integral_constant<int, 64>{});
+    if (t == 16) go(integral_constant<int, 16>{}, (void*)nullptr);
+    else if (t == 32) go(integral_constant<int, 32>{}, (void*)nullptr);
+    else if (t == 64) go(integral_constant<int, 64>{}, (void*)nullptr);
+    else if (t == 128) go(integral_constant<int, 128>{}, (void*)nullptr);
+    else if (f->n == 2 * MixedCt3840::M && mixed_plan_is(f->half, MixedCt3840::radix, MixedCt3840::count))
+        go(integral_constant<int, 256>{}, (MixedCt3840*)nullptr);
+    else go(integral_constant<int, 256>{}, (void*)nullptr);
 }
-size_t stft_frames_lds(int n) { return sizeof(float2) * ((size_t)kFrameJobs * frame_slot(n / 2) + n); }
-size_t istft_tile_lds(int n) { return stft_frames_lds(n) + sizeof(float) * n; }
+// Dynamic LDS: the frames' slots, the twiddles, and the fused iSTFT's window.
+template <int TPF>
+size_t frames_lds(int n, bool window) {
+    return sizeof(float2) * ((size_t)frame_jobs<TPF>() * frame_slot(n / 2) + (TPF <= 64 ? n : kMixedTwMax)) +
+           (window ? sizeof(float) * n : 0);
+}
 
-// Allows the kernels of this plan the CU's whole LDS (when the plan is created; the largest mixed-radix
-// n up to kFrameTw, 2000, takes 156.3 KB).
+// Allows the kernels of this plan the CU's whole LDS (when the plan is created; n_fft 2000 takes the most, 156.3 KB).
 void allow_frames_lds(const stx_fft* f) {
-    if (istft_tile_lds(f->n) <= 64 * 1024 || !frames_plan(f, kFrameMinJobs)) return;
-    pick_frame_threads(frames_plan(f, kFrameMinJobs), [&](auto tpf) {
+    const int t = frame_threads(f->n / 2, f->half);
+    if (!t) return;
+    auto allow = [](const void* k) {
+        hip_check(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024), "hipFuncSetAttribute");
+    };
+    pick_frame_threads(f, t, [&](auto tpf, auto* ct) {
         constexpr int TPF = decltype(tpf)::value;
-        const void* ks[2] = {reinterpret_cast<const void*>(stft_frames_kernel<TPF, kFrameJobs>),
-                             reinterpret_cast<const void*>(istft_tile_kernel<TPF, kFrameJobs>)};
-        for (const void* k : ks)
-            hip_check(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024), "hipFuncSetAttribute");
+        using CT = typename std::remove_pointer<decltype(ct)>::type;
+        if (frames_lds<TPF>(f->n, TPF <= 64) <= 64 * 1024) return;
+        allow(reinterpret_cast<const void*>(stft_frames_kernel<TPF, frame_jobs<TPF>(), CT>));
+        if constexpr (TPF <= 64) allow(reinterpret_cast<const void*>(istft_tile_kernel<TPF, kFrameJobs>));
+        else allow(reinterpret_cast<const void*>(istft_frames_kernel<TPF, frame_jobs<TPF>(), CT>));
     });
 }
 
 void launch_stft_frames(const stx_fft* f, StftArgs a, hipStream_t s) {
-    a.nblocks = (a.jobs + kFrameJobs - 1) / kFrameJobs;
-    const size_t lds = stft_frames_lds(f->n);
-    pick_frame_threads(frames_plan(f, a.jobs), [&](auto tpf) {
-        constexpr int TPF = decltype(tpf)::value;
-        hipLaunchKernelGGL((stft_frames_kernel<TPF, kFrameJobs>), dim3(xcd_grid(a.nblocks)), dim3(TPF * kFrameJobs), lds, s, a,
-                           f->half, f->twn, f->n, FastDiv((unsigned)a.T));
+    pick_frame_threads(f, frames_plan(f, a.jobs), [&](auto tpf, auto* ct) {
+        constexpr int TPF = decltype(tpf)::value, JOBS = frame_jobs<TPF>();
+        using CT = typename std::remove_pointer<decltype(ct)>::type;
+        a.nblocks = (a.jobs + JOBS - 1) / JOBS;
+        hipLaunchKernelGGL((stft_frames_kernel<TPF, JOBS, CT>), dim3(xcd_grid(a.nblocks)), dim3(TPF * JOBS),
+                           frames_lds<TPF>(f->n, false), s, a, f->half, f->twn, f->twm, f->n, FastDiv((unsigned)a.T));
     });
     launch_check("stft_frames_kernel");
 }
 
-// Tiles of m hops need m + ceil(n / hop) - 1 frames: m from the block's 16 frames.
-void launch_istft_tiles(const stx_fft* f, IstftArgs a, int channels, hipStream_t s) {
-    const int span = (f->n + a.hop - 1) / a.hop, m = kFrameJobs - span + 1;
-    a.tile_len = m * a.hop;
-    a.tile_origin = a.out_off - a.out_off % a.hop;
-    a.tiles = (int)(((long long)a.out_off + a.out_len - a.tile_origin + a.tile_len - 1) / a.tile_len);
-    a.nblocks = a.tiles * channels;
-    const size_t lds = istft_tile_lds(f->n);
-    pick_frame_threads(frames_plan(f, (long long)channels * a.T), [&](auto tpf) {
-        constexpr int TPF = decltype(tpf)::value;
-        hipLaunchKernelGGL((istft_tile_kernel<TPF, kFrameJobs>), dim3(xcd_grid(a.nblocks)), dim3(TPF * kFrameJobs), lds, s, a,
-                           f->half, f->twn, f->n, FastDiv((unsigned)a.hop), FastDiv((unsigned)a.tiles));
+// The iSTFT of many frames of a mixed-radix size; false where the call takes one frame a workgroup.
+// n <= kFrameTw: fused tiles of m hops, which need m + ceil(n / hop) - 1 frames, where at most half of a tile's
+// 16 frames are shared with the next. Larger n: the frames to the workspace, then their sums.
+bool launch_istft_frames(const stx_fft* f, IstftArgs a, int channels, hipStream_t s) {
+    const int t = frames_plan(f, (long long)channels * a.T);
+    if (!t) return false;
+    bool done = false;
+    pick_frame_threads(f, t, [&](auto tpf, auto* ct) {
+        constexpr int TPF = decltype(tpf)::value, JOBS = frame_jobs<TPF>();
+        using CT = typename std::remove_pointer<decltype(ct)>::type;
+        if constexpr (TPF <= 64) {
+            const int span = (f->n + a.hop - 1) / a.hop;
+            if (2 * span > JOBS) return;
+            a.tile_len = (JOBS - span + 1) * a.hop;
+            a.tile_origin = a.out_off - a.out_off % a.hop;
+            a.tiles = (int)(((long long)a.out_off + a.out_len - a.tile_origin + a.tile_len - 1) / a.tile_len);
+            a.nblocks = a.tiles * channels;
+            hipLaunchKernelGGL((istft_tile_kernel<TPF, JOBS>), dim3(xcd_grid(a.nblocks)), dim3(TPF * JOBS),
+                               frames_lds<TPF>(f->n, true), s, a, f->half, f->twn, f->n, FastDiv((unsigned)a.hop),
+                               FastDiv((unsigned)a.tiles));
+            launch_check("istft_tile_kernel");
+        } else {
+            const int groups = (a.T + JOBS - 1) / JOBS;
+            a.nblocks = groups * channels;
+            hipLaunchKernelGGL((istft_frames_kernel<TPF, JOBS, CT>), dim3(xcd_grid(a.nblocks)), dim3(TPF * JOBS),
+                               frames_lds<TPF>(f->n, false), s, a, f->half, f->twn, f->twm, f->n, groups, FastDiv((unsigned)groups));
+            launch_check("istft_frames_kernel");
+            hipLaunchKernelGGL(istft_ola_kernel, dim3((a.out_len + 255) / 256, channels), dim3(256), 0, s, a, f->n);
+            launch_check("istft_ola_kernel");
+        }
+        done = true;
     });
-    launch_check("istft_tile_kernel");
+    return done;
 }
 
 template <int N>
@@ -1465,12 +1574,8 @@ void run_istft(const stx_fft* f, IstftArgs a, int channels, void* workspace, siz
         const size_t need = istft_workspace_bytes(f->n, channels, a.T);
         STX_REQUIRE(ws_bytes >= need, "workspace too small: %zu bytes, need %zu", ws_bytes, need);
         check_extent((long long)channels * a.T * f->n, "workspace");
-        // At most half of a tile's frames shared with the next: the fused tiles.
-        if (frames_plan(f, (long long)channels * a.T) && 2 * ((f->n + a.hop - 1) / a.hop) <= kFrameJobs) {
-            launch_istft_tiles(f, a, channels, s);
-            return;
-        }
         a.frames = static_cast<float*>(workspace);
+        if (launch_istft_frames(f, a, channels, s)) return;
         const int jobs = channels * a.T;
         // Two frames per block where a bin's two frames are one aligned 16-byte load (f-major, T
         // even) and both frames' buffers fit in LDS (n / 2 <= 4096).

@@ -470,13 +470,18 @@ def test_mixed_pairs_unaligned_spectrum(device, n, hop, frames):
     assert np.array_equal(ya, yb)
 
 
-# n_fft with 8 .. 1,024 points in the half transform (16, 32 and 64 threads a frame, plans that start with radix 16
+# n_fft with 9 .. 1,000 points in the half transform (16, 32 and 64 threads a frame, plans that start with radix 16
 # and not, the limits 240 | 250, 480 | 486, 960 | 1,000), hops from n / 8 to n, ends inside a tile of 16 frames,
 # tiles and workgroups that cross channels, and frames just below and above the switch to them (1,024).
 FRAME_CASES = [(960, 480, 3, 1023 * 160 + 7), (320, 80, 2, 80 * 600 + 3), (320, 106, 1, 106 * 1024), (480, 60, 2, 60 * 700 + 59),
                (500, 125, 2, 125 * 530), (972, 243, 2, 243 * 520 + 1), (18, 9, 2, 9 * 900 + 4), (48, 48, 1, 48 * 1100),
                (640, 640, 2, 640 * 520), (1536, 512, 3, 512 * 400 + 100), (1920, 480, 2, 480 * 515), (2000, 500, 2, 500 * 512),
-               (2000, 250, 4, 250 * 256), (960, 240, 1, 240 * 1022), (960, 240, 1, 240 * 1023), (960, 100, 2, 100 * 520)]
+               (2000, 250, 4, 250 * 256), (960, 240, 1, 240 * 1022), (960, 240, 1, 240 * 1023), (960, 100, 2, 100 * 520),
+               # 128 and 256 threads a frame (above 512 frames): the compiled plan, plans that start with radix 15 and 8,
+               # 1,920 | 2,025 and 3,840 points, odd frame counts, a size that stays with one frame a workgroup (8100).
+               (7680, 1024, 3, 1024 * 255 + 9), (7680, 1920, 2, 1920 * 256), (7680, 1024, 2, 1024 * 255), (3840, 960, 2, 960 * 272),
+               (4050, 1350, 4, 1350 * 130 + 1), (6000, 1500, 3, 1500 * 200), (2160, 540, 3, 540 * 200 + 2), (8192 - 192, 1000, 3, 1000 * 180),
+               (6144, 6144, 3, 6144 * 180), (8100, 2025, 3, 2025 * 180)]
 
 
 @pytest.mark.parametrize("n,hop,channels,length", FRAME_CASES)
@@ -487,8 +492,9 @@ def test_mixed_many_frames(device, orc, n, hop, channels, length, layout):
     f = any_plan(n)
     T = length // hop + 1
     spec = stx.torch_stft(f, to_dev(x, device), hop, layout=layout)
-    ws = stx.workspace(stx.istft_workspace_size(f, channels, T), device)
+    ws = stx.workspace(stx.istft_workspace_size(f, channels, T) + 4, device)
     y = host(stx.torch_istft(f, spec, hop, layout=layout, workspace=ws))
+    assert np.array_equal(y, host(stx.torch_istft(f, spec, hop, layout=layout, workspace=ws[1:])))   # 4-byte aligned
     spec_h = host(spec)
     if layout == stx.T_MAJOR:
         spec_h = spec_h.transpose(0, 2, 1)
