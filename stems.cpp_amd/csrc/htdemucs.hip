@@ -494,14 +494,30 @@ __global__ __launch_bounds__(256) void cac_denorm_kernel(const float* ox, float2
 }
 
 // Time branch: out = (float)(t * sd + mean) + y, the add in float.
+// One float a thread; V4: four (16-byte aligned arrays), the last n % 4 by the first threads of the
+// last block (8 channels of a 343,980-sample segment, 33 MB: 9.4 -> 7.5 us).
+template <bool V4>
 __global__ __launch_bounds__(256) void time_add_kernel(const float* t, const float* y, float* out, long long n,
                                                        const double* stats) {
 #pragma clang fp contract(off)
     const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (e >= n) return;
     const double mean = stats[0], sd = stats[1];
-    const float a = (float)((double)t[e] * sd + mean);
-    store_stream(out + e, a + y[e]);
+    auto one = [&](float tv, float yv) {
+        const float a = (float)((double)tv * sd + mean);
+        return a + yv;
+    };
+    if constexpr (V4) {
+        const long long n4 = n / 4;
+        if (e < n4) {
+            const float4 a = reinterpret_cast<const float4*>(t)[e], b = reinterpret_cast<const float4*>(y)[e];
+            store_stream(reinterpret_cast<float4*>(out) + e, make_float4(one(a.x, b.x), one(a.y, b.y), one(a.z, b.z), one(a.w, b.w)));
+        } else if (e - n4 < n % 4) {
+            const long long i = 4 * n4 + (e - n4);
+            store_stream(out + i, one(t[i], y[i]));
+        }
+    } else if (e < n) {
+        store_stream(out + e, one(t[e], y[e]));
+    }
 }
 
 // ------------------------------------------------------------------------------- split
@@ -856,8 +872,13 @@ STX_API stx_status stx_htdemucs_time_add(const float* xt, const float* y, int64_
         STX_REQUIRE(xt && y && out && stats, "NULL buffer");
         const long long blocks = (n + 255) / 256;
         STX_REQUIRE(blocks < (1LL << 31), "time_add: too many elements");
-        hipLaunchKernelGGL(time_add_kernel, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), xt, y, out,
-                           (long long)n, stats);
+        const bool v4 = ((reinterpret_cast<uintptr_t>(xt) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
+        if (v4)
+            hipLaunchKernelGGL(time_add_kernel<true>, dim3((unsigned)((n / 4 + n % 4 + 255) / 256)), dim3(256), 0, as_stream(stream),
+                               xt, y, out, (long long)n, stats);
+        else
+            hipLaunchKernelGGL(time_add_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), xt, y, out,
+                               (long long)n, stats);
         launch_check("time_add_kernel");
     });
 }

@@ -233,6 +233,24 @@ def test_denormalize_and_time_add_c1(device, htd):
     assert np.array_equal(host(out), htd.time_add(host(xt), host(y), -0.002, 0.09))
 
 
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 7, 1023, 1024, 1025, 4099])
+@pytest.mark.parametrize("off", [(0, 0, 0), (1, 1, 1), (0, 1, 0), (0, 0, 3)])
+def test_time_add_sizes(device, htd, n, off):
+    """Counts around the four-float loads' ends, 16-byte aligned and not, and in place: the oracle's bits, nothing written past
+    the end."""
+    import torch
+    tstats = torch.tensor([-0.002, 0.09], dtype=torch.float64, device=device)
+    x, y = dev(synth.normal(6, (n + 4,), 1.0), device)[off[0]:off[0] + n], dev(synth.normal(7, (n + 4,), 1.0), device)[off[1]:off[1] + n]
+    buf = torch.full((n + 8,), 5.5, device=device)
+    want = htd.time_add(host(x), host(y), -0.002, 0.09)
+    stx.htdemucs_time_add(x, y, tstats, out=buf[off[2]:off[2] + n])
+    got = host(buf)
+    assert np.array_equal(got[off[2]:off[2] + n], want)
+    assert np.all(got[:off[2]] == 5.5) and np.all(got[off[2] + n:] == 5.5)
+    stx.htdemucs_time_add(x, y, tstats, out=y)
+    assert np.array_equal(host(y), want)
+
+
 @pytest.mark.parametrize("shifted", [False, True])
 def test_segments_song(device, htd, shifted):
     """TensorChunk views of the 180 s song: the plain split and one shift view (the mix padded
