@@ -585,7 +585,7 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_kernel(IstftArgs a) 
 // 5 hops, at 2048, 441 16 gave 12. T-major, 8 channels of an HTDemucs segment 49.4 -> 31.5 us, 32 RoFormer
 // channels 138 -> 109, 192 727 -> 565 (2.7 TB/s); n_fft 8192, hop 1024 250 -> 90. What is left per round of 16
 // frames at 2048 (16 us) is 10 us of VALU issue and the LDS round trips of passes whose waves move together;
-// two workgroups of 7 frames a CU measured slower (109 -> 152: 130 registers, 14 waves).
+// two workgroups of 7 frames a CU measured slower (109 -> 114).
 template <int N, int P, int JOBS>
 __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_run_kernel(IstftArgs a) {
     constexpr int M = N / 2;

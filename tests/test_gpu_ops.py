@@ -448,6 +448,41 @@ def test_add_mul_broadcast_bit_exact(device, ops, shape, bshape):
     assert np.array_equal(host(stx.mul(a, b)), ops.binary("mul", ah, bh))
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 1), (1, 1, 3), (5, 1, 205), (4, 1, 256), (3, 1, 1025), (7, 2, 293)])
+@pytest.mark.parametrize("off", [(0, 1), (1, 0), (3, 3)])
+def test_elementwise_unaligned(device, shape, off):
+    """Dense arrays that are not 16-byte aligned (scalar loads over the flat index) give the bits of aligned ones, for every
+    op and operand kind (same shape, per channel, per row, one value), in place and without writing past the end."""
+    import torch
+    n = int(np.prod(shape))
+
+    def at(k, seed, shape=shape):
+        m = int(np.prod(shape))
+        t = torch.zeros(m + 8, device=device)[k:k + m].view(shape)
+        t.copy_(randn(device, shape, seed))
+        return t
+
+    a, h, g = (at(off[0], k) for k in (1, 2, 3))
+    al = [t.clone() for t in (a, h, g)]
+    C = shape[0]
+    for bs in (shape, (C, 1, 1), (shape[-1],), (1,)):
+        b = randn(device, bs, 4)
+        for f in (stx.add, stx.mul):
+            out = torch.full((n + 8,), 5.5, device=device)
+            f(a, b, out=out[off[1]:off[1] + n].view(shape))
+            assert torch.equal(out[off[1]:off[1] + n].view(shape), f(al[0], b))
+            assert bool((out[:off[1]] == 5.5).all()) and bool((out[off[1] + n:] == 5.5).all())
+        assert torch.equal(stx.gelu_erf(a, b), stx.gelu_erf(al[0], b))
+        assert torch.equal(stx.mul_add(a, h, b, out=at(off[1], 5)), stx.mul_add(al[0], al[1], b))
+    assert torch.equal(stx.gelu_erf(a, out=at(off[1], 5)), stx.gelu_erf(al[0]))
+    two = (2 * C,) + tuple(shape[1:])
+    d, s = at(off[0], 6, two), randn(device, (C, 1, 1), 7)
+    assert torch.equal(stx.glu(d, 2, out=at(off[1], 5)), stx.glu(d.clone(), 2))
+    assert torch.equal(stx.glu_mul_add(a, d, 2, s, out=at(off[1], 5)), stx.glu_mul_add(al[0], d.clone(), 2, s))
+    want = stx.mul_add(al[0], al[1], s)
+    assert torch.equal(stx.mul_add(a, h, s, out=a), want)
+
+
 def test_binary_strided_views(device, ops):
     big = randn(device, (40, 3, 257), 25)
     a = big[:, 1, :]                                         # non-contiguous rows
