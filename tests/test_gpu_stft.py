@@ -477,6 +477,8 @@ FRAME_CASES = [(960, 480, 3, 1023 * 160 + 7), (320, 80, 2, 80 * 600 + 3), (320, 
                (500, 125, 2, 125 * 530), (972, 243, 2, 243 * 520 + 1), (18, 9, 2, 9 * 900 + 4), (48, 48, 1, 48 * 1100),
                (640, 640, 2, 640 * 520), (1536, 512, 3, 512 * 400 + 100), (1920, 480, 2, 480 * 515), (2000, 500, 2, 500 * 512),
                (2000, 250, 4, 250 * 256), (960, 240, 1, 240 * 1022), (960, 240, 1, 240 * 1023), (960, 100, 2, 100 * 520),
+               # Even hops whose output begins at an odd sample of the frames' grid (n / 2 odd).
+               (18, 6, 2, 6 * 1100 + 5), (50, 10, 3, 10 * 700), (810, 202, 2, 202 * 600 + 1),
                # 128 and 256 threads a frame (above 512 frames): the compiled plan, plans that start with radix 15 and 8,
                # 1,920 | 2,025 and 3,840 points, odd frame counts, a size that stays with one frame a workgroup (8100).
                (7680, 1024, 3, 1024 * 255 + 9), (7680, 1920, 2, 1920 * 256), (7680, 1024, 2, 1024 * 255), (3840, 960, 2, 960 * 272),
