@@ -247,6 +247,11 @@ struct IstftArgs {
     float norm;
 };
 
+// Where a tile ends. The last one's nominal end may pass 2^31.
+__device__ __forceinline__ int tile_end(const IstftArgs& a, int tile) {
+    return (int)min((unsigned)(a.out_off + a.out_len), (unsigned)a.tile_origin + ((unsigned)tile + 1) * (unsigned)a.tile_len);
+}
+
 __device__ __forceinline__ float2 spec_bin(const IstftArgs& a, const float2* __restrict__ sc, int st, int k) {
     return a.layout == STX_SPEC_F_MAJOR ? sc[(size_t)k * a.T + st] : sc[(size_t)st * a.F + k];
 }
@@ -463,7 +468,7 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_kernel(IstftArgs a) 
 
     const int c = lb / a.tiles, tile = lb - c * a.tiles;
     const int J0 = max(a.out_off, a.tile_origin + tile * a.tile_len);
-    const int J1 = min(a.out_off + a.out_len, a.tile_origin + (tile + 1) * a.tile_len);
+    const int J1 = tile_end(a, tile);
     // Spectrum frames overlapping [J0, J1): envelope frame tf covers [tf*hop, tf*hop + N).
     const int st_lo = max(0, max(0, ceildiv(J0 - N + 1, hop)) - a.frame_off);
     const int st_hi = min(a.T - 1, floordiv(J1 - 1, hop) - a.frame_off);
@@ -610,7 +615,7 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_run_kernel(IstftArgs
     const int hop = a.hop;
     const int c = lb / a.tiles, run = lb - c * a.tiles;
     const int J0 = max(a.out_off, a.tile_origin + run * a.tile_len);
-    const int J1 = min(a.out_off + a.out_len, a.tile_origin + (run + 1) * a.tile_len);
+    const int J1 = tile_end(a, run);
     const int K0 = (N - 1) / hop, rK = N - 1 - K0 * hop;
     const int clen = max(N - hop, 0);
     float* inv_env = tail;
@@ -1063,7 +1068,7 @@ __global__ __launch_bounds__(TPF * JOBS) __attribute__((amdgpu_waves_per_eu(4)))
     wins.load(a.win, n, tid);
     const int c = (int)ftiles.div((unsigned)lb), tile = lb - c * a.tiles;
     const int J0 = max(a.out_off, a.tile_origin + tile * a.tile_len);
-    const int J1 = min(a.out_off + a.out_len, a.tile_origin + (tile + 1) * a.tile_len);
+    const int J1 = tile_end(a, tile);
     const int st_lo = max(0, max(0, ceildiv(J0 - n + 1, a.hop)) - a.frame_off);
     const int st_hi = min(a.T - 1, floordiv(J1 - 1, a.hop) - a.frame_off);
     const float2* sc = a.spec + (size_t)c * a.T * a.F;
@@ -1092,8 +1097,9 @@ __global__ __launch_bounds__(TPF * JOBS) __attribute__((amdgpu_waves_per_eu(4)))
     if (hop % 2 == 0) {
         // Samples J and J + 1, J even, are the two halves of one element of every frame that covers them (n is even):
         // half the reads and index work. 960 / 480, 2 channels of 60 s: 38.1 -> 32.2 us; 1,536 / 384 of 45 s: 71.5 -> 62.6.
-        for (int J = (J0 & ~1) + 2 * tid; J < J1; J += 2 * NT) {
-            const int A = (int)fhop.div((unsigned)J), R = J - A * hop, K = R <= rK ? K0 : K0 - 1;
+        const int Je = J0 & ~1;
+        for (int x = 2 * tid; x < J1 - Je; x += 2 * NT) {
+            const int J = Je + x, A = (int)fhop.div((unsigned)J), R = J - A * hop, K = R <= rK ? K0 : K0 - 1;
             float s0 = 0.f, s1 = 0.f, e0 = 0.f, e1 = 0.f;
             for (int q = K; q >= 0; q--) {             // frame order
                 const int tf = A - q, st = tf - a.frame_off, pos = R + q * hop;
@@ -1113,8 +1119,8 @@ __global__ __launch_bounds__(TPF * JOBS) __attribute__((amdgpu_waves_per_eu(4)))
         }
         return;
     }
-    for (int J = J0 + tid; J < J1; J += NT) {
-        const int A = (int)fhop.div((unsigned)J), R = J - A * hop, K = R <= rK ? K0 : K0 - 1;
+    for (int x = tid; x < J1 - J0; x += NT) {
+        const int J = J0 + x, A = (int)fhop.div((unsigned)J), R = J - A * hop, K = R <= rK ? K0 : K0 - 1;
         float sum = 0.f, env = 0.f;
         for (int q = K; q >= 0; q--) {                 // frame order
             const int tf = A - q, st = tf - a.frame_off, pos = R + q * hop;
