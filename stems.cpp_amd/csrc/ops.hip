@@ -835,7 +835,7 @@ struct GroupNormArgs {
     int groups;              // groups per ne3 slice
     int nch;                 // chunks per group (of the largest group)
     float eps;
-    int vec;                 // every group span is 16-byte aligned and a multiple of 4 floats
+    int vec;                 // every group starts 16-byte aligned, and all but a ragged last one end so
 };
 
 __device__ __forceinline__ void group_span(const GroupNormArgs& a, int gt, long long& begin, unsigned& count,
@@ -1351,7 +1351,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void gn
             bl[i] = a.b.p ? a.b.p[c0 + i] : 0.f;
         }
     }
-    if (a.vec) gn_group_body<AFF, GELU, NT, K, true>(a, a.x + begin, a.y + begin, count, wl, bl, nc, red);
+    // a.vec speaks of the whole groups: a ragged last one may end inside a float4.
+    if (a.vec && count % 4 == 0) gn_group_body<AFF, GELU, NT, K, true>(a, a.x + begin, a.y + begin, count, wl, bl, nc, red);
     else gn_group_body<AFF, GELU, NT, K, false>(a, a.x + begin, a.y + begin, count, wl, bl, nc, red);
 }
 

@@ -230,6 +230,29 @@ def test_group_norm_many_groups_same_bits(device, ops, shape, G, along, gelu):
         assert np.array_equal(one, host(stx.group_norm(x, G, 1e-5, None, b.expand(plane).contiguous(), gelu=gelu)))
 
 
+# (ne2, groups, plane): cpg * plane is a multiple of 4, so the groups start 16-byte aligned, and the ragged last one has
+# 602, 302, 150, 6 and 2 floats; 2,050 floats past the first chunk; 300 (whole float4s).
+@pytest.mark.parametrize("ne2,G,plane", [(50, 16, 301), (19, 10, 302), (35, 18, 150), (19, 10, 6), (19, 10, 2), (19, 10, 2050),
+                                         (19, 10, 300)])
+@pytest.mark.parametrize("affine", [False, True])
+@pytest.mark.parametrize("gelu", [False, True])
+def test_group_norm_ragged_last_group(device, ops, ne2, G, plane, affine, gelu):
+    """One block per group where the last group has fewer channels and may end inside a float4: the oracle's values, the
+    general path's bits, and nothing written past the tensor."""
+    import torch
+    x = randn(device, (ne2, 1, plane), ne2 + plane, 1.3, 0.7)
+    w, b = (randn(device, (ne2, 1, 1), 70), randn(device, (ne2, 1, 1), 71)) if affine else (None, None)
+    buf = torch.full((x.numel() + 16,), 5.5, device=device)
+    stx.group_norm(x, G, 1e-5, w, b, gelu=gelu, out=buf[:x.numel()].view(x.shape))
+    y, guard = host(buf[:x.numel()].view(x.shape)), host(buf[x.numel():])
+    assert np.all(guard == 5.5)
+    want = ops.group_norm(host(x), G, 1e-5, host(w) if affine else None, host(b) if affine else None, gelu=gelu)
+    assert rel_err(y, want) <= TOL
+    if affine:
+        full = stx.group_norm(x, G, 1e-5, w.expand(ne2, 1, plane).contiguous(), b.expand(ne2, 1, plane).contiguous(), gelu=gelu)
+        assert np.array_equal(host(full), y)
+
+
 def test_group_norm_errors(device):
     import torch
     x = randn(device, (4, 1, 100), 10)
