@@ -564,7 +564,9 @@ typedef struct {
  *     fallback word (stx_grid_sync_fallbacks). Streams created with a CU mask, HSA_CU_MASK,
  *     ROC_GLOBAL_CU_MASK and STX_NO_GRID_SYNC=1 select the two-kernel path;
  *   - more than 8 groups of at most 65,536 floats, with parameters per channel (or, with one ne2
- *     index per group, per ne1 index) or none, run as one kernel with a block per group;
+ *     index per group, per ne1 index) or none, run as one kernel with a block per group where there
+ *     are enough of them for their size to fill the device (any number of groups of up to 4,096
+ *     floats, 128 groups of 64,512);
  *   - everything else runs as two kernels (three for groups of more than 2^23 floats). */
 STX_API size_t     stx_group_norm_workspace_size(const stx_tensor* a, int n_groups);
 STX_API stx_status stx_group_norm(const stx_tensor* a, const stx_tensor* dst, int n_groups, float eps,

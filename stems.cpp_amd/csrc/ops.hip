@@ -786,7 +786,7 @@ __global__ __launch_bounds__(256) void ew_flat1_kernel(const float* __restrict__
 //   single pass (gn_fused_kernel) when the groups fit on the device at once, VEC < 4 and y
 //     does not overlap x: x is read once, the blocks exchange their partial sums (grid_sync.hpp);
 //   one block per group (gn_group_kernel) for more than kGridMaxGroups groups of at most 65,536
-//     floats;
+//     floats, enough of them to fill the device (gn_group_least);
 //   two passes otherwise: gn_partial_kernel writes each chunk's partial sums (and K), then
 //     gn_apply_kernel folds its group's partials itself (or reads gn_fold_kernel's totals when
 //     a group has more than kGnFoldDirect chunks) and writes its chunk.
@@ -1707,12 +1707,31 @@ void launch_gn_vec(const GroupNormArgs& g, const GnPlan& p, const GridSync& sync
     launch_check("gn_apply_kernel");
 }
 
-// Launches gn_group_kernel where it applies: more groups than the single pass takes (few groups
-// are spread over more CUs by it), every group in one block's registers, affine per channel or none.
+// Chunks of a launch from which on a block per group beats the two passes, for groups of nch chunks. A block takes as
+// long as its group is, however few there are (128 groups of 4,096 floats 3.9 us, of 32,768 14.7, of 65,536 23.5; with
+// GELU 4.8, 20.8 and 35.8); the two passes take 5.5 us and their bytes, spread over every CU. Group kernel / two passes
+// in us, planes of 336 or 512 floats, parameters per channel:
+//   12,096 floats: 96 groups 7.7 / 8.7, 64 7.3 / 7.5
+//   32,768: 512 groups 27.3 / 39.8; 32,256: 128 14.5 / 15.2, 112 14.3 / 13.9, 64 13.5 / 10.2; 32,768: 9 12.3 / 5.7
+//   64,512: 512 groups 55.3 / 82.7, 128 23.1 / 24.5, 112 22.7 / 22.0, 9 20.6 / 6.8
+// and with GELU
+//   8,064: 96 groups 7.2 / 8.7, 64 6.8 / 6.8; 8,192: 96 6.7 / 7.6, 64 6.7 / 6.2; 16,128: 112 groups 11.6 / 11.7
+//   32,256: 176 groups 21.7 / 22.5, 144 21.0 / 19.5; 64,512: 160 groups 35.4 / 36.7, 128 34.2 / 29.8
+inline long long gn_group_least(int nch, bool gelu) {
+    if (nch <= 2) return 0;
+    if (nch <= 4) return gelu ? 300 : 0;
+    if (nch <= 8) return gelu ? 900 : 450;
+    if (nch <= 16) return gelu ? 2600 : 2000;
+    return gelu ? 4700 : 3700;
+}
+
+// Launches gn_group_kernel where it applies: more groups than the single pass takes, enough of them for their size,
+// every group in one block's registers, affine per channel or none.
 template <bool GELU>
 bool launch_gn_groups(const GroupNormArgs& g, const GnPlan& p, int ak, bool disjoint, hipStream_t s) {
     const bool aff = g.w.p || g.b.p;
     if (p.groups_total <= kGridMaxGroups || p.nch > kGnGroupMaxChunks || p.vec != 1 || !(disjoint || g.x == g.y)) return false;
+    if (p.groups_total * p.nch < gn_group_least(p.nch, GELU)) return false;
     if (aff && ((ak != AFF_CHANNEL && ak != AFF_CHANNEL_WAVE) || g.cpg > kGnGroupMaxChannels || g.plane < 4)) return false;
     auto go = [&](auto affine, auto threads, auto chunks) {
         constexpr bool A = decltype(affine)::value;

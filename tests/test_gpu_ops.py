@@ -197,14 +197,19 @@ def test_group_norm_paths_same_bits(device, ops, shape, G, gelu, monkeypatch):
         assert forced > 0
 
 
-# (torch shape, groups, parameters along): one group per block up to 32 chunks of 2,048 floats, its limits
+# (torch shape, groups, parameters along): one block per group up to 32 chunks of 2,048 floats, its limits
 # (32,768 | 32,769.. | 65,536 | 65,568 floats, 1,024 | 1,025 channels, planes of 4 | 3 floats), unaligned
 # spans, a ragged last group, a batch, and 8 groups (the grid-synchronised pass).
 GN_GROUP_CASES = [((512, 6, 336), 512, "ne1"), ((20, 96, 336), 20, "ne1"), ((9, 16, 2048), 9, "ne1"), ((9, 331, 99), 9, "ne1"),
                   ((10, 128, 512), 10, "ne1"), ((10, 96, 683), 10, "ne1"), ((33, 5, 333), 33, "ne1"), ((9, 1024, 5), 9, "ne1"),
                   ((9, 1025, 5), 9, "ne1"), ((16, 7, 4), 16, "ne1"), ((16, 7, 3), 16, "ne1"), ((11, 1, 1), 11, "ne1"),
                   ((8, 96, 336), 8, "ne1"), ((2, 6, 48, 85), 6, "ne1"), ((64, 1, 700), 16, "ne2"), ((47, 1, 301), 10, "ne2"),
-                  ((3, 14, 2, 130), 4, "ne2"), ((12, 3, 1000), 12, "none")]
+                  ((3, 14, 2, 130), 4, "ne2"), ((12, 3, 1000), 12, "none"),
+                  # Groups of 4 | 5, 8, 9, 16 | 17, 32 chunks in the numbers that take a block per group, with GELU and without
+                  # (300, 900, 2,600, 4,700 chunks), and one group fewer (one block per group without GELU, two passes with it).
+                  ((75, 16, 512), 75, "ne1"), ((74, 16, 512), 74, "ne1"), ((180, 17, 512), 180, "ne1"), ((113, 33, 489), 113, "ne1"),
+                  ((112, 32, 512), 112, "ne2"), ((289, 17, 1001), 289, "ne1"), ((163, 16, 2048), 163, "ne1"),
+                  ((162, 96, 336), 162, "none"), ((277, 331, 99), 277, "ne1"), ((147, 128, 512), 147, "ne1"), ((146, 192, 336), 146, "ne1")]
 
 
 @pytest.mark.parametrize("shape,G,along", GN_GROUP_CASES)
