@@ -570,7 +570,8 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_kernel(IstftArgs a) 
         const int J = J0 + q * NT + tid;
         if (J >= J1) return;
         float y = 0.f;
-        if (ENV_LDS && J < a.valid_end && tf0 >= 0 && tf0 + K < a.env_frames) {
+        // K < 0: between frames (hop > N), past the table; env_quotient gives 0 there.
+        if (ENV_LDS && K >= 0 && J < a.valid_end && tf0 >= 0 && tf0 + K < a.env_frames) {
             const float r = inv_env[s_first - K * hop];
             y = r > 0.f ? acc[q] * r : 0.f;
         } else if (J < a.valid_end) {
@@ -674,7 +675,7 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_run_kernel(IstftArgs
                     const float sum = frames_at(x, A, R, F > F0 && x < clen ? carry[x] : 0.f);
                     const int K = R <= rK ? K0 : K0 - 1, tf0 = F + A - K;
                     float y = 0.f;
-                    if (J < a.valid_end && tf0 >= 0 && tf0 + K < a.env_frames) {
+                    if (K >= 0 && J < a.valid_end && tf0 >= 0 && tf0 + K < a.env_frames) {   // as in istft_kernel
                         const float r = inv_env[R];
                         y = r > 0.f ? sum * r : 0.f;
                     } else if (J < a.valid_end) {

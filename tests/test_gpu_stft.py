@@ -327,6 +327,33 @@ def test_istft_runs(device, orc, layout, n, hop, length, channels):
         assert np.array_equal(y[c], y[0])
 
 
+# Hops above n_fft: samples between the frames that no frame covers. Calls of a few tiles and of more than the device holds
+# workgroups; an odd number of channels, one sample uncovered (n + 1) and most of them.
+GAP_CASES = [(2048, 2049, 6, 2), (2048, 3000, 5, 1), (2048, 5001, 400, 3), (1024, 1500, 900, 2), (512, 20000, 100, 3), (16, 40, 30, 2),
+             (16, 41, 300001, 1), (64, 1000, 4001, 1), (8192, 10000, 300, 2), (4096, 4097, 500, 3)]
+
+
+@pytest.mark.parametrize("layout", [stx.F_MAJOR, stx.T_MAJOR])
+@pytest.mark.parametrize("n,hop,frames,channels", GAP_CASES)
+def test_istft_hop_above_n(device, layout, n, hop, frames, channels):
+    """Frames that do not meet: a covered sample is its frame's own inverse (over the window, as w^2 / w^2), so the frames of
+    one call laid n apart (hop n, whose oracle comparisons are test_istft_runs') have the same bits; an uncovered one is 0."""
+    x = synth.normal(4600 + n + hop, (channels, frames * n), 0.2)
+    f = plan(n)
+    spec = stx.torch_stft(f, to_dev(x, device), n, layout=layout)
+    T = frames + 1                                           # length // n + 1
+    y = host(stx.torch_istft(f, spec, hop, layout=layout))
+    close = host(stx.torch_istft(f, spec, n, layout=layout))
+    assert y.shape == (channels, hop * (T - 1))
+    # Signal index J of sample i is i + n / 2; frame t covers [t hop, t hop + n).
+    J = np.arange(y.shape[1]) + n // 2
+    R = J % hop
+    assert np.all(y[:, R >= n] == 0.0)
+    covered = (J // hop) * n + R - n // 2
+    sel = (R < n) & (covered < close.shape[1]) & (covered >= 0)
+    assert np.array_equal(y[:, sel], close[:, covered[sel]])
+
+
 def test_istft_many_tiles_graph_replays(device):
     """A captured torch_istft call whose tiles outnumber the resident workgroups, replayed on new
     spectra with eager work between the replays: every replay equals the eager call's bits."""
