@@ -591,7 +591,7 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_kernel(IstftArgs a) 
 // 5 hops, at 2048, 441 16 gave 12. T-major, 8 channels of an HTDemucs segment 49.4 -> 31.5 us, 32 RoFormer
 // channels 138 -> 109, 192 727 -> 565 (2.7 TB/s); n_fft 8192, hop 1024 250 -> 90. What is left per round of 16
 // frames at 2048 (16 us) is 10 us of VALU issue and the LDS round trips of passes whose waves move together;
-// two workgroups of 7 frames a CU measured slower (109 -> 114).
+// two workgroups of 7 frames a CU measured slower (109 -> 114). Hops up to N only (launch_istft_fused).
 template <int N, int P, int JOBS>
 __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_run_kernel(IstftArgs a) {
     constexpr int M = N / 2;
@@ -604,8 +604,8 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_run_kernel(IstftArgs
     __shared__ float2 lds[JOBS * SLOT];
     __shared__ float2 twt[TwTable<N>::SIZE];
     __shared__ float wl[N];
-    // [0, min(hop, N)): reciprocal envelope per position R = J mod hop where every covering frame
-    // exists; then the carry (N - hop samples; none for hop >= N).
+    // [0, hop), hop <= N: reciprocal envelope per position R = J mod hop where every covering frame
+    // exists; then the carry (N - hop samples).
     __shared__ float tail[N];
     const int lb = xcd_block();
     if (lb >= a.nblocks) return;
@@ -618,9 +618,9 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_run_kernel(IstftArgs
     const int J0 = max(a.out_off, a.tile_origin + run * a.tile_len);
     const int J1 = tile_end(a, run);
     const int K0 = (N - 1) / hop, rK = N - 1 - K0 * hop;
-    const int clen = max(N - hop, 0);
+    const int clen = N - hop;
     float* inv_env = tail;
-    float* carry = tail + min(hop, N);
+    float* carry = tail + hop;
     // Envelope frames F0 .. F1 reach into [J0, J1).
     const int F0 = J0 / hop - K0, F1 = (J1 - 1) / hop;
     const SpecStage<N, P, JOBS, SLOT> io{a, a.spec + (size_t)c * a.T * a.F, lds, a.T - 1};
@@ -635,7 +635,7 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_run_kernel(IstftArgs
     wins.store(wl, tid);
     lds_barrier();
     const WindowMul post{reinterpret_cast<const float2*>(wl)};
-    for (int R = tid; R < min(hop, N); R += NT) {      // read after the first round's barriers
+    for (int R = tid; R < hop; R += NT) {              // read after the first round's barriers
         float env = 0.f;
         for (int i = R <= rK ? K0 : K0 - 1; i >= 0; i--) {
             const float w = wl[R + i * hop];
@@ -675,7 +675,7 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_run_kernel(IstftArgs
                     const float sum = frames_at(x, A, R, F > F0 && x < clen ? carry[x] : 0.f);
                     const int K = R <= rK ? K0 : K0 - 1, tf0 = F + A - K;
                     float y = 0.f;
-                    if (K >= 0 && J < a.valid_end && tf0 >= 0 && tf0 + K < a.env_frames) {   // as in istft_kernel
+                    if (J < a.valid_end && tf0 >= 0 && tf0 + K < a.env_frames) {
                         const float r = inv_env[R];
                         y = r > 0.f ? sum * r : 0.f;
                     } else if (J < a.valid_end) {
@@ -1434,8 +1434,10 @@ void launch_istft_fused(IstftArgs a, int channels, hipStream_t s) {
             return;
         }
     }
+    // Hops above N share no frames between tiles, and most of their samples are zeros: tiles of kIstftPer samples a thread
+    // spread the stores over the device, where a run of JOBS hops leaves them to one workgroup.
     IstftArgs t = a;
-    if (plan_istft_tiles<N, JOBS>(t, channels) > istft_resident<N, JOBS>()) launch_istft_runs<N>(a, channels, s);
+    if (a.hop <= N && plan_istft_tiles<N, JOBS>(t, channels) > istft_resident<N, JOBS>()) launch_istft_runs<N>(a, channels, s);
     else launch_istft_fused_jobs<N, JOBS>(a, channels, s);
 }
 

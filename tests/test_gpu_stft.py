@@ -330,7 +330,9 @@ def test_istft_runs(device, orc, layout, n, hop, length, channels):
 # Hops above n_fft: samples between the frames that no frame covers. Calls of a few tiles and of more than the device holds
 # workgroups; an odd number of channels, one sample uncovered (n + 1) and most of them.
 GAP_CASES = [(2048, 2049, 6, 2), (2048, 3000, 5, 1), (2048, 5001, 400, 3), (1024, 1500, 900, 2), (512, 20000, 100, 3), (16, 40, 30, 2),
-             (16, 41, 300001, 1), (64, 1000, 4001, 1), (8192, 10000, 300, 2), (4096, 4097, 500, 3)]
+             (16, 41, 300001, 1), (64, 1000, 4001, 1), (8192, 10000, 300, 2), (4096, 4097, 500, 3),
+             # Hops whose product with the frames of a workgroup (512 at n_fft 16) passes 2^31.
+             (16, 5000000, 2, 2), (16, 4194305, 4, 1), (32, 10000000, 3, 1)]
 
 
 @pytest.mark.parametrize("layout", [stx.F_MAJOR, stx.T_MAJOR])
