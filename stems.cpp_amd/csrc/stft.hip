@@ -1504,7 +1504,10 @@ void launch_stft_frames(const stx_fft* f, StftArgs a, hipStream_t s) {
 
 // The iSTFT of many frames of a mixed-radix size; false where the call takes one frame a workgroup.
 // n <= kFrameTw: fused tiles of m hops, which need m + ceil(n / hop) - 1 frames, where at most half of a tile's
-// 16 frames are shared with the next. Larger n: the frames to the workspace, then their sums.
+// 16 frames are shared with the next. Hops of several n are mostly zeros, which 16 hops a workgroup leave to few
+// workgroups: above 4 n the two kernels, whose sums spread over the device (n_fft 320, 1,100 frames: hop 640 21 us
+// as two kernels, 15 as tiles; 1,600 24 and 21; 6,400 33 and 51; 32,000 79 and 203). Larger n: the frames to the
+// workspace, then their sums.
 bool launch_istft_frames(const stx_fft* f, IstftArgs a, int channels, hipStream_t s) {
     const int t = frames_plan(f, (long long)channels * a.T);
     if (!t) return false;
@@ -1514,7 +1517,7 @@ bool launch_istft_frames(const stx_fft* f, IstftArgs a, int channels, hipStream_
         using CT = typename std::remove_pointer<decltype(ct)>::type;
         if constexpr (TPF <= 64) {
             const int span = (f->n + a.hop - 1) / a.hop;
-            if (2 * span > JOBS) return;
+            if (2 * span > JOBS || a.hop / 4 > f->n) return;
             a.tile_len = (JOBS - span + 1) * a.hop;
             a.tile_origin = a.out_off - a.out_off % a.hop;
             a.tiles = (int)(((long long)a.out_off + a.out_len - a.tile_origin + a.tile_len - 1) / a.tile_len);

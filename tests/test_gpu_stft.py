@@ -515,6 +515,27 @@ FRAME_CASES = [(960, 480, 3, 1023 * 160 + 7), (320, 80, 2, 80 * 600 + 3), (320, 
                (6144, 6144, 3, 6144 * 180), (8100, 2025, 3, 2025 * 180)]
 
 
+# Hops of 4 n and less (fused tiles) and above (two kernels), for calls of many frames.
+@pytest.mark.parametrize("n,hop,frames", [(320, 1280, 1100), (320, 1284, 1100), (960, 1500, 1030), (96, 9600, 1025), (2000, 9001, 1600)])
+@pytest.mark.parametrize("layout", [stx.F_MAJOR, stx.T_MAJOR])
+def test_mixed_istft_hop_above_n(device, n, hop, frames, layout):
+    """Frames that do not meet: the samples that a frame covers against the same frames laid n apart, the others 0. Both
+    sum one windowed frame and divide by the window's square; the transforms' plan is the same at both hops."""
+    x = synth.normal(4700 + n + hop, (1, frames * n), 0.2)
+    f = any_plan(n)
+    spec = stx.torch_stft(f, to_dev(x, device), n, layout=layout)
+    ws = stx.workspace(stx.istft_workspace_size(f, 1, frames + 1), device)
+    y = host(stx.torch_istft(f, spec, hop, layout=layout, workspace=ws))
+    close = host(stx.torch_istft(f, spec, n, layout=layout, workspace=ws))
+    J = np.arange(y.shape[1]) + n // 2
+    R = J % hop
+    assert np.all(y[:, R >= n] == 0.0)
+    covered = (J // hop) * n + R - n // 2
+    sel = (R < n) & (covered < close.shape[1]) & (covered >= 0)
+    w = 0.5 - 0.5 * np.cos(2.0 * np.pi * R[sel] / n)         # a sample is w x / w^2: compare w y, the frame
+    assert snr_db(y[:, sel] * w, close[:, covered[sel]] * w) >= SNR_DB
+
+
 @pytest.mark.parametrize("n,hop,channels,length", FRAME_CASES)
 @pytest.mark.parametrize("layout", [stx.F_MAJOR, stx.T_MAJOR])
 def test_mixed_many_frames(device, orc, n, hop, channels, length, layout):
