@@ -1442,17 +1442,34 @@ void launch_istft_fused(IstftArgs a, int channels, hipStream_t s) {
 }
 
 // The several-frames kernels' workgroups: 16 frames of frame_threads() threads (16, 32 or 64; n <= kFrameTw), 4 of
-// 128 or 2 of 256. 0: not for this plan or this many frames (channels times frames): with few, one frame a
-// workgroup of 512 threads is faster. Up to 64 threads below about 1,024 frames (n_fft 960, 368 frames: 8.7 against
-// 9.6 us, iSTFT 11.9 against 13.6; 11,026 frames: 120 against 23, iSTFT 143 against 35); 128 and 256 up to the two
-// frames a CU that those workgroups hold at once (n_fft 7680 f-major, 512 frames: 16.6 against 16.4 and 23.7 against
-// 24.5 us; 768: 25.5 against 19.7, 35.9 against 28.6).
+// 128 or 2 of 256. 0: not for this plan or this many frames (channels times frames), where one frame a workgroup of
+// 512 threads is faster, as measured in us (one frame against several):
+//   - Up to 64 threads, plans that start with radix 16: from kFrameMinJobs frames on. n_fft 960, 368 frames: 8.7 against
+//     9.6, iSTFT 11.9 against 13.6; 1,920 t-major, 1,024 frames: equal; 11,026 frames of 960: 120 against 23, 143 against 35.
+//     Other plans take more passes of small radices: n_fft 2000 (8 x 5 x 5 x 5) t-major, 1,024 frames 14.3 against 20.5,
+//     1,400 equal within 6 %, 1,600 21.4 against 20.1; 1,944, 1,458 and 1,296 cross there too.
+//   - 128 and 256 threads: from the two frames a CU on that those workgroups hold at once (n_fft 7680 f-major, 512
+//     frames: 16.6 against 16.4, iSTFT 23.7 against 24.5; 768: 25.5 against 19.7, 35.9 against 28.6; 5,120 and 6,144 alike).
+//     256 threads and a plan without radix 16 (4,050, 4,374, 6,250, 7,290): from 3 frames a CU, t-major rows from 5
+//     (7,290 t-major, 600 frames: 9 % slower, 1,200 6 %, 1,300 5 % faster).
+//   - n_fft 7680's iSTFT of t-major rows between 4 and 5 frames a CU (the second round of workgroups nearly empty): 1,100
+//     frames 36.6 against 38.4, where 1,024 take 32.0 against 29.9 and 1,300 40.9 against 40.6.
 constexpr int kFrameJobs = 16;
 constexpr int kFrameMinJobs = 1024;
+constexpr int kFrameMinJobsOther = 1536;
 template <int TPF> constexpr int frame_jobs() { return TPF <= 64 ? kFrameJobs : TPF == 128 ? 4 : 2; }
-int frames_plan(const stx_fft* f, long long jobs) {
+bool compiled_plan(const stx_fft* f) {
+    return f->n == 2 * MixedCt3840::M && mixed_plan_is(f->half, MixedCt3840::radix, MixedCt3840::count);
+}
+int frames_plan(const stx_fft* f, long long jobs, int layout, bool inverse) {
     const int t = frame_threads(f->n / 2, f->half);
-    return jobs >= (t <= 64 ? kFrameMinJobs : 2LL * device_cus() + 1) ? t : 0;
+    const bool radix16 = f->half.r[0] == 16, rows = layout == STX_SPEC_T_MAJOR;
+    const long long cus = device_cus();
+    if (inverse && rows && jobs > 4 * cus && jobs <= 5 * cus && compiled_plan(f)) return 0;
+    long long least = 2 * cus + 1;
+    if (t <= 64) least = radix16 ? kFrameMinJobs : kFrameMinJobsOther;
+    else if (t == 256 && !radix16) least = (rows ? 5 : 3) * cus + 1;
+    return jobs >= least ? t : 0;
 }
 
 // Calls go(integral_constant<int, TPF>, CT*) for t threads a frame, CT the compiled plan of n_fft 7680 or void.
@@ -1463,8 +1480,7 @@ void pick_frame_threads(const stx_fft* f, int t, F&& go) {
     else if (t == 32) go(integral_constant<int, 32>{}, (void*)nullptr);
     else if (t == 64) go(integral_constant<int, 64>{}, (void*)nullptr);
     else if (t == 128) go(integral_constant<int, 128>{}, (void*)nullptr);
-    else if (f->n == 2 * MixedCt3840::M && mixed_plan_is(f->half, MixedCt3840::radix, MixedCt3840::count))
-        go(integral_constant<int, 256>{}, (MixedCt3840*)nullptr);
+    else if (compiled_plan(f)) go(integral_constant<int, 256>{}, (MixedCt3840*)nullptr);
     else go(integral_constant<int, 256>{}, (void*)nullptr);
 }
 // Dynamic LDS: the frames' slots, the twiddles, and the fused iSTFT's window.
@@ -1492,7 +1508,7 @@ void allow_frames_lds(const stx_fft* f) {
 }
 
 void launch_stft_frames(const stx_fft* f, StftArgs a, hipStream_t s) {
-    pick_frame_threads(f, frames_plan(f, a.jobs), [&](auto tpf, auto* ct) {
+    pick_frame_threads(f, frames_plan(f, a.jobs, a.layout, false), [&](auto tpf, auto* ct) {
         constexpr int TPF = decltype(tpf)::value, JOBS = frame_jobs<TPF>();
         using CT = typename std::remove_pointer<decltype(ct)>::type;
         a.nblocks = (a.jobs + JOBS - 1) / JOBS;
@@ -1509,7 +1525,7 @@ void launch_stft_frames(const stx_fft* f, StftArgs a, hipStream_t s) {
 // as two kernels, 15 as tiles; 1,600 24 and 21; 6,400 33 and 51; 32,000 79 and 203). Larger n: the frames to the
 // workspace, then their sums.
 bool launch_istft_frames(const stx_fft* f, IstftArgs a, int channels, hipStream_t s) {
-    const int t = frames_plan(f, (long long)channels * a.T);
+    const int t = frames_plan(f, (long long)channels * a.T, a.layout, true);
     if (!t) return false;
     bool done = false;
     pick_frame_threads(f, t, [&](auto tpf, auto* ct) {
@@ -1620,7 +1636,7 @@ void run_istft(const stx_fft* f, IstftArgs a, int channels, void* workspace, siz
         const int blocks = pair ? jobs / 2 : jobs;
         const unsigned grid = (unsigned)((blocks + kXcds - 1) / kXcds * kXcds);   // xcd_block's multiple
         const dim3 bd(kMixedThreads * (pair ? 2 : 1));
-        const bool ct = f->n == 2 * MixedCt3840::M && mixed_plan_is(f->half, MixedCt3840::radix, MixedCt3840::count);
+        const bool ct = compiled_plan(f);
         if (ct && pair)
             hipLaunchKernelGGL((istft_frames_mixed_kernel<4096, MixedCt3840, 2>), dim3(grid), bd, 0, s, a, f->half, f->twn,
                                f->twm, f->n, jobs);
@@ -1958,7 +1974,7 @@ STX_API stx_status stx_torch_stft(const stx_fft* f, const float* x, int channels
         a.win_hs = f->win_hs ? f->win_hs + (normalized ? n : 0) : nullptr;
         check_extent((long long)channels * a.T * a.F, "spectrum");
         check_extent((long long)channels * len + n, "signal");
-        if (f->mixed && frames_plan(f, a.jobs)) {
+        if (f->mixed && frames_plan(f, a.jobs, a.layout, false)) {
             launch_stft_frames(f, a, as_stream(stream));
             return;
         }
@@ -1971,7 +1987,7 @@ STX_API stx_status stx_torch_stft(const stx_fft* f, const float* x, int channels
             const unsigned grid = (unsigned)((blocks + kXcds - 1) / kXcds * kXcds);   // xcd_block's multiple
             const dim3 bd(kMixedThreads * (pair ? 2 : 1));
             const hipStream_t st = as_stream(stream);
-            const bool ct = n == 2 * MixedCt3840::M && mixed_plan_is(f->half, MixedCt3840::radix, MixedCt3840::count);
+            const bool ct = compiled_plan(f);
             if (ct && pair)
                 hipLaunchKernelGGL((stft_mixed_kernel<4096, MixedCt3840, 2>), dim3(grid), bd, 0, st, a, f->half, f->twn,
                                    f->twm, n);

@@ -501,7 +501,8 @@ def test_mixed_pairs_unaligned_spectrum(device, n, hop, frames):
 
 # n_fft with 9 .. 1,000 points in the half transform (16, 32 and 64 threads a frame, plans that start with radix 16
 # and not, the limits 240 | 250, 480 | 486, 960 | 1,000), hops from n / 8 to n, ends inside a tile of 16 frames,
-# tiles and workgroups that cross channels, and frames just below and above the switch to them (1,024).
+# tiles and workgroups that cross channels, and frames just below and above the switch to them (1,024 where the plan
+# starts with radix 16).
 FRAME_CASES = [(960, 480, 3, 1023 * 160 + 7), (320, 80, 2, 80 * 600 + 3), (320, 106, 1, 106 * 1024), (480, 60, 2, 60 * 700 + 59),
                (500, 125, 2, 125 * 530), (972, 243, 2, 243 * 520 + 1), (18, 9, 2, 9 * 900 + 4), (48, 48, 1, 48 * 1100),
                (640, 640, 2, 640 * 520), (1536, 512, 3, 512 * 400 + 100), (1920, 480, 2, 480 * 515), (2000, 500, 2, 500 * 512),
@@ -512,7 +513,13 @@ FRAME_CASES = [(960, 480, 3, 1023 * 160 + 7), (320, 80, 2, 80 * 600 + 3), (320, 
                # 1,920 | 2,025 and 3,840 points, odd frame counts, a size that stays with one frame a workgroup (8100).
                (7680, 1024, 3, 1024 * 255 + 9), (7680, 1920, 2, 1920 * 256), (7680, 1024, 2, 1024 * 255), (3840, 960, 2, 960 * 272),
                (4050, 1350, 4, 1350 * 130 + 1), (6000, 1500, 3, 1500 * 200), (2160, 540, 3, 540 * 200 + 2), (8192 - 192, 1000, 3, 1000 * 180),
-               (6144, 6144, 3, 6144 * 180), (8100, 2025, 3, 2025 * 180)]
+               (6144, 6144, 3, 6144 * 180), (8100, 2025, 3, 2025 * 180),
+               # Plans that do not start with radix 16 on both sides of their own switch: 1,536 frames up to 64 threads a frame,
+               # 768 (f-major) and 1,280 (t-major) with 256; n_fft 7680 where its t-major iSTFT takes one frame a workgroup.
+               (500, 125, 2, 125 * 766), (500, 125, 2, 125 * 767), (972, 243, 2, 243 * 780 + 1), (18, 9, 2, 9 * 1500 + 4),
+               (18, 6, 2, 6 * 1600 + 5), (810, 202, 2, 202 * 800 + 1), (2000, 500, 2, 500 * 800), (2000, 250, 4, 250 * 400),
+               (1350, 450, 2, 450 * 790), (4050, 1350, 3, 1350 * 255), (4050, 1350, 3, 1350 * 256), (4050, 1350, 4, 1350 * 330 + 1),
+               (6000, 1500, 4, 1500 * 330), (7290, 2430, 5, 2430 * 257), (7680, 1024, 4, 1024 * 270), (7680, 1920, 4, 1920 * 330)]
 
 
 # Hops of 4 n and less (fused tiles) and above (two kernels), for calls of many frames.
