@@ -1321,19 +1321,34 @@ void launch_stft_jobs(StftArgs a, hipStream_t s) {
 }
 
 // Frames per workgroup. Few frames: one in the T-major layout (the most workgroups), two in the
-// F-major layout, whose bins then leave as 16-byte runs of two frames per row instead of 8. From
-// kStftMany frames on, when they fill the device several times over, F-major rows take runs of four
+// F-major layout, whose bins then leave as 16-byte runs of two frames per row instead of 8. Calls of
+// many frames, when they fill the device several times over (stft_many): F-major rows take runs of four
 // frames (32 stereo chunks at n_fft 2048, hop 441: 115 -> 84 us; 8 frames 96), short frames of either
 // layout eight and 1,024-point frames in rows of their own four (n_fft 128, hop 64, 62,502 frames: 29 -> 16 us,
 // T-major 48 -> 23; n_fft 1024: 54 -> 42, 39 -> 36).
-constexpr int kStftMany = 2048;
+// The lines, few frames a workgroup against many in us: from 2,048 frames on, except
+//   - 512 f-major from 3,328 (2,050 frames 6.1 / 6.6, 3,000 7.1 / 7.2, 3,584 7.7 / 7.4);
+//   - 2048 f-major from 2,560 (2,178 frames 12.8 / 13.6, 2,562 16.6 / 14.0);
+//   - 1024 t-major from 8,192 (2,050 frames 7.2 / 7.6, 6,144 11.7 / 11.7, 14,000 by 5 %);
+//   - 4096 f-major, whose workgroups of four frames are 1,024 threads, two a CU: not where a nearly empty last round of
+//     them follows one or two full ones (2,048 frames 22.0 / 19.7, 2,050 21.7 / 26.2, 2,562 27.1 / 26.9, 3,000 28.5 /
+//     26.3, 4,500 38.0 / 40.0, 6,000 48.2 / 42.7, 14,000 138 / 109).
+template <int N>
+bool stft_many(const StftArgs& a) {
+    if (a.layout == STX_SPEC_T_MAJOR) return a.jobs >= (N == 1024 ? 8192 : 2048);
+    if (N == 4096) {
+        const int round = 8 * device_cus();
+        return a.jobs >= round && (a.jobs > 4 * round || (a.jobs - 1) % round >= round / 4);
+    }
+    return a.jobs >= (N == 512 ? 3328 : N == 2048 ? 2560 : 2048);
+}
 
 template <int N>
 void launch_stft(const StftArgs& a, hipStream_t s) {
     constexpr int TPJ = N / 2 / kStftP;
     constexpr bool SHORT = N <= 512;
     constexpr int J2 = TPJ * 2 <= 1024 ? 2 : 1, FMANY = SHORT ? 8 : TPJ * 4 <= 1024 ? 4 : J2, TMANY = SHORT ? 8 : N == 1024 ? 4 : 1;
-    const bool many = a.jobs >= kStftMany;
+    const bool many = stft_many<N>(a);
     if (a.layout == STX_SPEC_T_MAJOR) {
         if (TMANY > 1 && many) launch_stft_jobs<N, TMANY>(a, s);
         else launch_stft_jobs<N, 1>(a, s);

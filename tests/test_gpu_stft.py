@@ -278,12 +278,15 @@ def test_htdemucs_ispec_many_segments_same_bits_as_pairs(device, orc, layout):
         assert snr_db(y[c], orc.htdemucs_ispec(ref, 4096, length)) >= SNR_DB
 
 
-# The switch to several frames a workgroup (2,048 frames), the last workgroup partly past the end and workgroups that
-# cross channels, for every group size (8, 4 and 1).
+# The switch to several frames a workgroup (2,048 frames; 512 f-major 3,328, 2048 f-major 2,560, 1024 t-major 8,192, 4096
+# f-major by how full its last round of workgroups is), the last workgroup partly past the end and workgroups that cross
+# channels, for every group size (8, 4 and 1).
 @pytest.mark.parametrize("layout", [stx.F_MAJOR, stx.T_MAJOR])
 @pytest.mark.parametrize("n,hop,length,channels", [(2048, 441, 441 * 1025, 2), (2048, 441, 441 * 682 + 3, 3), (1024, 256, 256 * 410 + 9, 5),
                                                    (512, 128, 128 * 1026, 2), (128, 64, 64 * 2049 + 1, 1), (16, 4, 4 * 1030, 2),
-                                                   (8192, 2048, 2048 * 420, 5), (4096, 1024, 1024 * 684, 3)])
+                                                   (8192, 2048, 2048 * 420, 5), (4096, 1024, 1024 * 684, 3),
+                                                   (2048, 441, 441 * 870 + 5, 3), (512, 128, 128 * 1110 + 3, 3), (1024, 256, 256 * 1640, 5),
+                                                   (4096, 1024, 1024 * 861 + 1, 3), (4096, 1024, 1024 * 1023, 2)])
 def test_stft_many_frames(device, orc, layout, n, hop, length, channels):
     """STFT calls of 2,048 frames and more: every channel has the bits of a call of its own (fewer frames, one or two a
     workgroup), and the oracle's values."""
