@@ -1405,10 +1405,10 @@ constexpr int istft_run_jobs() {
 
 // Runs for calls with more tiles than the device holds workgroups: R rounds of JOBS frames give R JOBS -
 // K0 hops. R is the one whose workgroups (one or two a CU) take the fewest rounds in all, a workgroup's tables
-// and first loads counted as half a round.
+// and first loads counted as half a round. Returns twice those rounds.
 template <int N>
-void launch_istft_runs(IstftArgs a, int channels, hipStream_t s) {
-    constexpr int P = fused_p(N), JOBS = istft_run_jobs<N>();
+long long plan_istft_runs(IstftArgs& a, int channels) {
+    constexpr int JOBS = istft_run_jobs<N>();
     const long long K0 = (N - 1) / a.hop, cus = (long long)device_cus() * (1024 / istft_run_threads(N));
     const int A0 = a.out_off / a.hop;
     const long long hops = (a.out_off + (long long)a.out_len - 1) / a.hop - A0 + 1;
@@ -1428,6 +1428,27 @@ void launch_istft_runs(IstftArgs a, int channels, hipStream_t s) {
     a.tile_origin = A0 * a.hop;
     a.tiles = (int)((hops + best_hops - 1) / best_hops);
     a.nblocks = a.tiles * channels;
+    return best;
+}
+
+// Whether a call of `tiles` tiles (plan_istft_tiles in t) takes runs (runs: twice their rounds). T-major: always. F-major
+// rounds read 8 JOBS bytes of each row, and neighbouring tiles on one XCD share those lines while runs, which move along
+// their own rows, do not; so from n_fft 1024 to 4096 runs are taken where they save rounds (at 4096 their rounds have 7
+// frames, the tiles' 8). Tiles / runs in us, 4096 / 1024 f-major: 2,429 frames 37 / 35, 3,382 54 / 59, 3,991 69 / 62, 4,710 70 /
+// 82, 5,558 86 / 88, 7,739 121 / 112; 2048 / 441: 5,558 33 / 36, 6,558 47 / 39, 9,132 48 / 54, 15,005 78 / 74; t-major, the
+// same calls of 4096: 34 / 31, 51 / 45, 65 / 47, 67 / 60, 83 / 61, 113 / 76.
+template <int N, int JOBS>
+bool istft_runs_gain(const IstftArgs& t, long long tiles, long long runs) {
+    if (t.layout == STX_SPEC_T_MAJOR || N < 1024 || N > 4096) return true;
+    const long long span = t.tile_len % t.hop == 0 ? t.tile_len / t.hop + (N - 1) / t.hop : (t.tile_len + N - 2) / t.hop + 1;
+    const long long resident = istft_resident<N, JOBS>();
+    const long long rounds = (tiles + resident - 1) / resident * ((span + JOBS - 1) / JOBS);
+    return runs * JOBS <= 2 * rounds * istft_run_jobs<N>();
+}
+
+template <int N>
+void launch_istft_runs(const IstftArgs& a, hipStream_t s) {
+    constexpr int P = fused_p(N), JOBS = istft_run_jobs<N>();
     hipLaunchKernelGGL((istft_run_kernel<N, P, JOBS>), dim3(xcd_grid(a.nblocks)), dim3(JOBS * (N / 2 / P)), 0, s, a);
     launch_check("istft_run_kernel");
 }
@@ -1451,9 +1472,12 @@ void launch_istft_fused(IstftArgs a, int channels, hipStream_t s) {
     }
     // Hops above N share no frames between tiles, and most of their samples are zeros: tiles of kIstftPer samples a thread
     // spread the stores over the device, where a run of JOBS hops leaves them to one workgroup.
-    IstftArgs t = a;
-    if (a.hop <= N && plan_istft_tiles<N, JOBS>(t, channels) > istft_resident<N, JOBS>()) launch_istft_runs<N>(a, channels, s);
-    else launch_istft_fused_jobs<N, JOBS>(a, channels, s);
+    IstftArgs t = a, r = a;
+    const long long tiles = plan_istft_tiles<N, JOBS>(t, channels);
+    if (a.hop <= N && tiles > istft_resident<N, JOBS>() && istft_runs_gain<N, JOBS>(t, tiles, plan_istft_runs<N>(r, channels)))
+        launch_istft_runs<N>(r, s);
+    else
+        launch_istft_fused_jobs<N, JOBS>(a, channels, s);
 }
 
 // The several-frames kernels' workgroups: 16 frames of frame_threads() threads (16, 32 or 64; n <= kFrameTw), 4 of

@@ -258,8 +258,8 @@ def test_istft_more_tiles_than_resident_workgroups(device, orc, layout, n, hop, 
 
 @pytest.mark.parametrize("layout", [stx.F_MAJOR, stx.T_MAJOR])
 def test_htdemucs_ispec_many_segments_same_bits_as_pairs(device, orc, layout):
-    # 16 HTDemucs segments (n_fft 4096) in one call: 1,088 tiles of 5 hops, so runs of rounds of 7
-    # frames; a call of two segments takes 6-frame tiles of 3 hops, one per
+    # 16 HTDemucs segments (n_fft 4096) in one call: 1,088 tiles of 5 hops, t-major runs of rounds of
+    # 7 frames; a call of two segments takes 6-frame tiles of 3 hops, one per
     # workgroup. Each sample adds the same frames in the same order either way, so every
     # channel must come out bit for bit the same.
     length, channels = 343980, 16
@@ -304,8 +304,9 @@ def test_stft_many_frames(device, orc, layout, n, hop, length, channels):
 
 # Runs of istft_run_kernel at its edges: n_fft 8192 (two frames a round, the carry longer than a round finishes), hop n
 # (no carry), hops that leave one sample uncovered (n - 1) or divide nothing, one sample past a run's end, and every
-# power of two from 16 (many frames a round).
-RUN_CASES = [(8192, 1024, 1024 * 400 + 5, 3), (8192, 333, 333 * 500, 2), (4096, 1023, 1023 * 700 + 1, 2), (2048, 2048, 2048 * 500, 9),
+# power of two from 16 (many frames a round); 4096 f-major where runs save rounds (1,300 frames) and where tiles stay.
+RUN_CASES = [(8192, 1024, 1024 * 400 + 5, 3), (8192, 333, 333 * 500, 2), (4096, 1023, 1023 * 700 + 1, 2), (4096, 1024, 1024 * 1299, 2),
+             (4096, 1024, 1024 * 1570 + 3, 3), (2048, 2048, 2048 * 500, 9),
              (2048, 2047, 2047 * 700, 5), (1024, 300, 300 * 9001, 2), (512, 128, 128 * 17000 + 3, 2), (256, 64, 64 * 20001, 2),
              (128, 50, 50 * 30001, 2), (64, 16, 16 * 70001, 1), (32, 8, 8 * 400001, 1), (16, 4, 4 * 400001, 1)]
 
