@@ -567,8 +567,8 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_kernel(IstftArgs a) 
     }
     float* oc = a.out + (size_t)c * a.out_len;
     walk(tid, [&](int q, int tf0, int s_first, int K) {
+        if (q * NT + tid >= J1 - J0) return;            // J0 + a whole tile may pass 2^31
         const int J = J0 + q * NT + tid;
-        if (J >= J1) return;
         float y = 0.f;
         // K < 0: between frames (hop > N), past the table; env_quotient gives 0 there.
         if (ENV_LDS && K >= 0 && J < a.valid_end && tf0 >= 0 && tf0 + K < a.env_frames) {
@@ -669,9 +669,10 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_run_kernel(IstftArgs
         };
         {
             int A = tr / hop, R = tr - A * hop;
-            for (int x = tr; x < done; x += NT) {
+            const int left = J1 - F * hop;             // samples to the run's end: F hop + done may pass 2^31
+            for (int x = tr; x < min(done, left); x += NT) {
                 const int J = F * hop + x;
-                if (J >= J0 && J < J1) {
+                if (J >= J0) {
                     const float sum = frames_at(x, A, R, F > F0 && x < clen ? carry[x] : 0.f);
                     const int K = R <= rK ? K0 : K0 - 1, tf0 = F + A - K;
                     float y = 0.f;

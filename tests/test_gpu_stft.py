@@ -382,6 +382,26 @@ def test_istft_hop_above_n(device, layout, n, hop, frames, channels):
     assert np.array_equal(y[:, sel], close[:, covered[sel]])
 
 
+def test_istft_output_near_2_31(device):
+    """An output whose last tile starts less than a whole tile below 2^31 (8.6 GB): the frames' samples have the bits of the
+    same frames 3,000 apart, and nothing else is written but zeros."""
+    import torch
+    n, hop, near, T = 16, 2147483, 3000, 1001
+    f = plan(n)
+    g = torch.Generator(device=device)
+    g.manual_seed(31)
+    spec = torch.randn((1, n // 2 + 1, T), generator=g, device=device, dtype=torch.complex64)
+    out = torch.full((hop * (T - 1) + 64,), 5.5, device=device)
+    stx.torch_istft(f, spec, hop, out=out[:hop * (T - 1)].view(1, -1))
+    small = stx.torch_istft(f, spec, near)[0]
+    k = torch.arange(n, device=device) - n // 2
+    t = torch.arange(T, device=device)[:, None]
+    ok = (t * near + k >= 0) & (t * near + k < small.numel())
+    assert torch.equal(out[(t * hop + k)[ok]], small[(t * near + k)[ok]])
+    assert bool((out[hop * (T - 1):] == 5.5).all())
+    assert int(torch.count_nonzero(out[:hop * (T - 1)])) == int(torch.count_nonzero(small))
+
+
 def test_istft_many_tiles_graph_replays(device):
     """A captured torch_istft call whose tiles outnumber the resident workgroups, replayed on new
     spectra with eager work between the replays: every replay equals the eager call's bits."""
