@@ -566,12 +566,14 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_kernel(IstftArgs a) 
         lds_barrier();
     }
     float* oc = a.out + (size_t)c * a.out_len;
+    // Hops above N have samples between the frames, past the table: all of them take env_quotient, which gives those 0.
+    const int table_frames = hop <= N ? a.env_frames : -1;
     walk(tid, [&](int q, int tf0, int s_first, int K) {
-        if (q * NT + tid >= J1 - J0) return;            // J0 + a whole tile may pass 2^31
-        const int J = J0 + q * NT + tid;
+        const unsigned Ju = (unsigned)J0 + (unsigned)(q * NT + tid);   // J0 and a whole tile may pass 2^31
+        if (Ju >= (unsigned)J1) return;
+        const int J = (int)Ju;
         float y = 0.f;
-        // K < 0: between frames (hop > N), past the table; env_quotient gives 0 there.
-        if (ENV_LDS && K >= 0 && J < a.valid_end && tf0 >= 0 && tf0 + K < a.env_frames) {
+        if (ENV_LDS && J < a.valid_end && tf0 >= 0 && tf0 + K < table_frames) {
             const float r = inv_env[s_first - K * hop];
             y = r > 0.f ? acc[q] * r : 0.f;
         } else if (J < a.valid_end) {
