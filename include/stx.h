@@ -422,10 +422,11 @@ STX_API int64_t    stx_resample_length(const stx_resampler* resampler, int64_t n
  * which differ from the reference's per-output weights by the rounding of its position i / ratio:
  * measured within 2.0e-7 of the output's rms, 167 dB SNR, on 180 s of stereo at 48 kHz.
  * STX_RESAMPLE_EXACT=1 in the environment (read at each call) selects the per-tap kernel,
- * bit-identical to the reference (double sums in its order). That kernel is also used when the
- * phase path does not fit: more than 2^18 phase-table weights, or 16 periods of the ratio (dst / gcd
- * outputs each) whose input exceeds the device's LDS per workgroup. Equal rates copy. More than 8
- * channels is UNSUPPORTED. */
+ * bit-identical to the reference (double sums in its order). That kernel is also used for inputs of
+ * one or two channels shorter than half the filter's window (36 samples at 48 -> 44.1 kHz; stereo
+ * three quarters of that), and when the phase path does not fit: more than 2^18 phase-table weights,
+ * or 16 periods of the ratio (dst / gcd outputs each) whose input exceeds the device's LDS per
+ * workgroup. Equal rates copy. More than 8 channels is UNSUPPORTED. */
 STX_API stx_status stx_resample(const stx_resampler* resampler, const float* in, int channels, int64_t n, float* out,
                                 stx_stream stream);
 

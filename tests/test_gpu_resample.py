@@ -95,7 +95,8 @@ def test_resample_nonfinite(device, rs, src, dst, C, n, monkeypatch):
 @pytest.mark.parametrize("src,dst,C,n", [(48000, 16000, 2, 70001), (88200, 44100, 1, 5000), (44100, 88200, 2, 16 * 64 + 1),
                                          (32000, 44100, 1, 32 * 320 - 1), (96000, 8000, 2, 30011), (8000, 96000, 1, 2049),
                                          (11025, 48000, 3, 16 * 147), (48000, 44100, 8, 500001), (44100, 48000, 1, 16 * 147 + 1),
-                                         (48000, 32000, 1, 1), (96000, 8000, 1, 13), (44100, 44101, 1, 3001)])
+                                         (48000, 32000, 1, 1), (96000, 8000, 1, 13), (44100, 44101, 1, 3001),
+                                         (192000, 44100, 1, 5000), (192000, 44100, 2, 1001), (48000, 11025, 1, 200000)])
 def test_resample_ratios(device, rs, src, dst, C, n):
     """The default kernel against the oracle, within the bounds of test_resample_parity; then with a NaN, an infinity
     and a -infinity, which reach exactly the outputs whose windows hold them."""
@@ -114,6 +115,23 @@ def test_resample_ratios(device, rs, src, dst, C, n):
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
     fin = np.isfinite(want)
     assert float(np.max(np.abs(got[fin].astype(np.float64) - want[fin]))) <= 1e-6 * rms
+
+
+@pytest.mark.parametrize("src,dst", [(48000, 44100), (44100, 8000), (44100, 88200), (192000, 44100)])
+@pytest.mark.parametrize("C", [1, 2, 3])
+def test_resample_short_inputs(device, rs, src, dst, C):
+    """Mono inputs up to half a window and stereo ones up to 3/4 of that take the per-tap kernel (bit-exact); one sample more,
+    and three channels, the phase kernel."""
+    half = 32 / (0.95 * min(1.0, dst / src))
+    limit = int(half * (1.0 if C == 1 else 0.75))
+    r = stx.Resampler(src, dst)
+    for n in (limit // 2, limit, limit + 1):
+        x = synth.normal(n + C, (C, n), 0.3)
+        want, got = rs(x, src, dst), host(r(dev(x, device)))
+        rms = max(float(np.sqrt(np.mean(want.astype(np.float64) ** 2))), 1e-3)
+        assert float(np.max(np.abs(got.astype(np.float64) - want))) <= 1e-6 * rms
+        if n <= limit and C <= 2:
+            assert np.array_equal(got, want)
 
 
 def test_equal_rates_copy(device):
