@@ -1492,8 +1492,9 @@ void launch_istft_fused(IstftArgs a, int channels, hipStream_t s) {
 //     1,400 equal within 6 %, 1,600 21.4 against 20.1; 1,944, 1,458 and 1,296 cross there too.
 //   - 128 and 256 threads: from the two frames a CU on that those workgroups hold at once (n_fft 7680 f-major, 512
 //     frames: 16.6 against 16.4, iSTFT 23.7 against 24.5; 768: 25.5 against 19.7, 35.9 against 28.6; 5,120 and 6,144 alike).
-//     256 threads and a plan without radix 16 (4,050, 4,374, 6,250, 7,290): from 3 frames a CU, t-major rows from 5
-//     (7,290 t-major, 600 frames: 9 % slower, 1,200 6 %, 1,300 5 % faster).
+//     256 threads and a plan without radix 16 (4,050, 4,374, 6,250, 7,290): f-major from 2.5 frames a CU (4,374, 515
+//     frames: 6 % slower, 701 2 % slower iSTFT and 10 % faster STFT), t-major from 5 (7,290, 600 frames: 9 % slower,
+//     1,200 6 %, 1,300 5 % faster).
 //   - n_fft 7680's iSTFT of t-major rows between 4 and 5 frames a CU (the second round of workgroups nearly empty): 1,100
 //     frames 36.6 against 38.4, where 1,024 take 32.0 against 29.9 and 1,300 40.9 against 40.6.
 constexpr int kFrameJobs = 16;
@@ -1510,7 +1511,7 @@ int frames_plan(const stx_fft* f, long long jobs, int layout, bool inverse) {
     if (inverse && rows && jobs > 4 * cus && jobs <= 5 * cus && compiled_plan(f)) return 0;
     long long least = 2 * cus + 1;
     if (t <= 64) least = radix16 ? kFrameMinJobs : kFrameMinJobsOther;
-    else if (t == 256 && !radix16) least = (rows ? 5 : 3) * cus + 1;
+    else if (t == 256 && !radix16) least = (rows ? 5 * cus : 5 * cus / 2) + 1;
     return jobs >= least ? t : 0;
 }
 

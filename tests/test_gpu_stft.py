@@ -561,10 +561,10 @@ FRAME_CASES = [(960, 480, 3, 1023 * 160 + 7), (320, 80, 2, 80 * 600 + 3), (320, 
                (4050, 1350, 4, 1350 * 130 + 1), (6000, 1500, 3, 1500 * 200), (2160, 540, 3, 540 * 200 + 2), (8192 - 192, 1000, 3, 1000 * 180),
                (6144, 6144, 3, 6144 * 180), (8100, 2025, 3, 2025 * 180),
                # Plans that do not start with radix 16 on both sides of their own switch: 1,536 frames up to 64 threads a frame,
-               # 768 (f-major) and 1,280 (t-major) with 256; n_fft 7680 where its t-major iSTFT takes one frame a workgroup.
+               # 640 (f-major) and 1,280 (t-major) with 256; n_fft 7680 where its t-major iSTFT takes one frame a workgroup.
                (500, 125, 2, 125 * 766), (500, 125, 2, 125 * 767), (972, 243, 2, 243 * 780 + 1), (18, 9, 2, 9 * 1500 + 4),
                (18, 6, 2, 6 * 1600 + 5), (810, 202, 2, 202 * 800 + 1), (2000, 500, 2, 500 * 800), (2000, 250, 4, 250 * 400),
-               (1350, 450, 2, 450 * 790), (4050, 1350, 3, 1350 * 255), (4050, 1350, 3, 1350 * 256), (4050, 1350, 4, 1350 * 330 + 1),
+               (1350, 450, 2, 450 * 790), (4050, 1350, 2, 1350 * 319), (4050, 1350, 3, 1350 * 256), (4050, 1350, 4, 1350 * 330 + 1),
                (6000, 1500, 4, 1500 * 330), (7290, 2430, 5, 2430 * 257), (7680, 1024, 4, 1024 * 270), (7680, 1920, 4, 1920 * 330)]
 
 
