@@ -836,6 +836,7 @@ struct GroupNormArgs {
     int nch;                 // chunks per group (of the largest group)
     float eps;
     int vec;                 // every group starts 16-byte aligned, and all but a ragged last one end so
+    int odd_group;           // with vec: the ragged last group if it ends inside a float4, else -1
 };
 
 __device__ __forceinline__ void group_span(const GroupNormArgs& a, int gt, long long& begin, unsigned& count,
@@ -1351,8 +1352,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void gn
             bl[i] = a.b.p ? a.b.p[c0 + i] : 0.f;
         }
     }
-    // a.vec speaks of the whole groups: a ragged last one may end inside a float4.
-    if (a.vec && count % 4 == 0) gn_group_body<AFF, GELU, NT, K, true>(a, a.x + begin, a.y + begin, count, wl, bl, nc, red);
+    if (a.vec && (int)blockIdx.x != a.odd_group) gn_group_body<AFF, GELU, NT, K, true>(a, a.x + begin, a.y + begin, count, wl, bl, nc, red);
     else gn_group_body<AFF, GELU, NT, K, false>(a, a.x + begin, a.y + begin, count, wl, bl, nc, red);
 }
 
@@ -1708,15 +1708,15 @@ void launch_gn_vec(const GroupNormArgs& g, const GnPlan& p, const GridSync& sync
 }
 
 // Chunks of a launch from which on a block per group beats the two passes, for groups of nch chunks. A block takes as
-// long as its group is, however few there are (128 groups of 4,096 floats 3.9 us, of 32,768 14.7, of 65,536 23.5; with
-// GELU 4.8, 20.8 and 35.8); the two passes take 5.5 us and their bytes, spread over every CU. Group kernel / two passes
+// long as its group is, however few there are (128 groups of 4,096 floats 3.9 us, of 32,768 13.9, of 65,536 23.4; with
+// GELU 4.8, 21.0 and 36.0); the two passes take 5.5 us and their bytes, spread over every CU. Group kernel / two passes
 // in us, planes of 336 or 512 floats, parameters per channel:
-//   12,096 floats: 96 groups 7.7 / 8.7, 64 7.3 / 7.5
-//   32,768: 512 groups 27.3 / 39.8; 32,256: 128 14.5 / 15.2, 112 14.3 / 13.9, 64 13.5 / 10.2; 32,768: 9 12.3 / 5.7
-//   64,512: 512 groups 55.3 / 82.7, 128 23.1 / 24.5, 112 22.7 / 22.0, 9 20.6 / 6.8
+//   12,096 floats: 96 groups 7.7 / 8.8, 64 7.3 / 7.8, 9 6.8 / 5.9
+//   32,768: 512 groups 25.6 / 39.4, 128 13.9 / 13.8, 96 13.2 / 11.9, 9 12.2 / 5.6
+//   64,512: 512 groups 55.5 / 81.7, 128 23.1 / 25.0, 112 22.6 / 22.3, 9 20.5 / 6.8
 // and with GELU
-//   8,064: 96 groups 7.2 / 8.7, 64 6.8 / 6.8; 8,192: 96 6.7 / 7.6, 64 6.7 / 6.2; 16,128: 112 groups 11.6 / 11.7
-//   32,256: 176 groups 21.7 / 22.5, 144 21.0 / 19.5; 64,512: 160 groups 35.4 / 36.7, 128 34.2 / 29.8
+//   8,064: 96 groups 7.2 / 8.8, 64 6.6 / 6.8; 8,192: 64 6.6 / 6.5; 16,128: 112 groups 11.7 / 11.9, 96 11.6 / 10.7
+//   32,256: 176 groups 22.0 / 22.5, 144 21.4 / 19.5; 64,512: 160 groups 35.7 / 36.9, 128 35.0 / 30.1
 inline long long gn_group_least(int nch, bool gelu) {
     if (nch <= 2) return 0;
     if (nch <= 4) return gelu ? 300 : 0;
@@ -1804,6 +1804,9 @@ void group_norm(const stx_tensor* a, const stx_tensor* dst, int n_groups, float 
                     (p.groups_total == g.groups || (g.ne2 * (long long)g.plane) % 4 == 0)
                 ? 1
                 : 0;
+    // Found here: with `count % 4` in the kernel, known in its body, two values of the 16 float4 spilled (the frequency
+    // branch's DConv, 512 rows: 82.0 -> 85.4 us).
+    g.odd_group = (g.ne2 - (g.groups - 1) * g.cpg) * (long long)g.plane % 4 != 0 ? (int)p.groups_total - 1 : -1;
     const size_t nbytes = (size_t)nelem(ta) * 4;
     const bool single = !overlaps(ta.data, nbytes, td.data, nbytes);
     auto fits = [&](int kind) {
