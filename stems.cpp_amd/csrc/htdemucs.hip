@@ -494,8 +494,8 @@ __global__ __launch_bounds__(256) void cac_denorm_kernel(const float* ox, float2
 }
 
 // Time branch: out = (float)(t * sd + mean) + y, the add in float.
-// One float a thread; V4: four (16-byte aligned arrays), the last n % 4 by the first threads of the
-// last block (8 channels of a 343,980-sample segment, 33 MB: 9.4 -> 7.5 us).
+// One float a thread; V4: four (16-byte aligned arrays), the last n % 4 by the threads after the last
+// whole float4 (8 channels of a 343,980-sample segment, 33 MB: 9.4 -> 7.5 us).
 template <bool V4>
 __global__ __launch_bounds__(256) void time_add_kernel(const float* t, const float* y, float* out, long long n,
                                                        const double* stats) {

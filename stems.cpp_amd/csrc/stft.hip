@@ -12,15 +12,17 @@
 //     frames that touch no padding skip it;
 //   * the inverse transform is the forward one on conjugated data (ifft(X) = conj fft conj X),
 //     after the inverse split Z' = (X[k] + conj X[N/2-k]) + i W_N^-k (X[k] - conj X[N/2-k]);
-//   * the iSTFT overlap-add is in gather form, without atomics, in one of two ways:
-//       - fused (no workspace): one workgroup owns a tile of output samples (several tiles in
-//         turn when they outnumber the workgroups the device holds), inverse-transforms every
-//         frame that overlaps it (frames shared by two tiles are transformed by both), sums the
-//         windowed frames in frame order in registers and divides by the window-squared
-//         envelope, evaluated in closed form per sample;
+//   * the iSTFT overlap-add is in gather form, without atomics, in one of three ways:
+//       - tiles (istft_kernel, no workspace): one workgroup owns a tile of output samples,
+//         inverse-transforms every frame that overlaps it (frames shared by two tiles are
+//         transformed by both), sums the windowed frames in frame order in registers and divides
+//         by the window-squared envelope, evaluated in closed form per sample;
+//       - runs (istft_run_kernel, calls with more tiles than the device holds at once): one
+//         workgroup owns a run of hops of a channel and transforms each frame once, round after
+//         round, carrying the sums of the samples that the next round finishes in LDS;
 //       - two kernels (the mixed-radix sizes with a large n or few frames, with a workspace of
 //         C*T*N floats): one inverse-transforms each frame once and writes it windowed to the
-//         workspace, the next sums and divides. Power-of-two sizes run the fused kernel with or
+//         workspace, the next sums and divides. Power-of-two sizes run tiles or runs with or
 //         without a workspace (measured faster at every size), mixed-radix calls with many frames
 //         of n <= 2048 a fused one of their own (istft_tile_kernel).
 #include <algorithm>
@@ -591,9 +593,9 @@ __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_kernel(IstftArgs a) 
 // round's spectrum loads are in flight through a round's transform (its barriers wait for LDS only).
 // Tiles of JOBS frames transformed ceil(N / hop) - 1 of them twice: at n_fft 4096, hop 1024 8 frames gave
 // 5 hops, at 2048, 441 16 gave 12. T-major, 8 channels of an HTDemucs segment 49.4 -> 31.5 us, 32 RoFormer
-// channels 138 -> 109, 192 727 -> 565 (2.7 TB/s); n_fft 8192, hop 1024 250 -> 90. What is left per round of 16
-// frames at 2048 (16 us) is 10 us of VALU issue and the LDS round trips of passes whose waves move together;
-// two workgroups of 7 frames a CU measured slower (109 -> 114). Hops up to N only (launch_istft_fused).
+// channels 138 -> 109, 192 727 -> 565 (2.7 TB/s); n_fft 8192, hop 1024 250 -> 90. What is left, by counters, per
+// round of 16 frames at 2048 (15.8 us): 8.8 us of VALU issue, 5 us of the CU's LDS, and a third of the wave time in
+// waits, passes whose waves move together; two workgroups of 7 frames a CU measured slower (109 -> 114). Hops up to N only (launch_istft_fused).
 template <int N, int P, int JOBS>
 __global__ __launch_bounds__(JOBS * (N / 2 / P)) void istft_run_kernel(IstftArgs a) {
     constexpr int M = N / 2;
@@ -901,12 +903,14 @@ __global__ __launch_bounds__(kMixedThreads * FPB) void istft_frames_mixed_kernel
 // half transform of n_fft 960 has 480 points, 30 radix-16 butterflies, so a workgroup of 512 threads per
 // frame (stft_mixed_kernel) left 94 % of them idle, and in the f-major layout each frame owns 8
 // bytes of a row; JOBS = 16 frames make runs of 128. With TPF <= 64 a frame is one wave's, so its
-// passes need no barrier. The twiddles are the full table of W_n^m in LDS for n <= 2048. Bound by LDS
-// traffic and VALU issue: n_fft 960, hop 480, a minute of stereo f-major 120 -> 24.9 us (3.4 TB/s of the
-// signal and the spectrum), iSTFT 143 -> 32.2; n_fft 320, hop 80, 12,502 frames 95 -> 15.3 and 109 -> 17.2.
+// passes need no barrier. The twiddles are the full table of W_n^m in LDS for n <= 2048. Bound by VALU
+// issue: n_fft 960, hop 480, a minute of stereo f-major 120 -> 24.9 us (2.55 TB/s of the signal and the
+// spectrum; 14.8 us of it VALU issue, 5.7 the CU's LDS), iSTFT 143 -> 32.2 (24.3 and 7.3); n_fft 320, hop 80, 12,502 frames 95 -> 15.3 and 109 -> 17.2.
 // With 128 and 256 threads a frame (n up to 7680 and 8192) the passes have barriers, and what counts is the one LDS
 // buffer a frame: two workgroups of 2 frames a CU, where stft_mixed_kernel's two ping-pong buffers held 2 frames in
-// all. n_fft 7680, 2,048 frames f-major: STFT 53 -> 40 us, iSTFT 71 -> 61; 4 frames a workgroup 42 and 63.
+// all. n_fft 7680, 2,048 frames f-major: STFT 53 -> 39 us (23 of them VALU issue, 42 % of the wave time in waits),
+// iSTFT 71 -> 57; 4 frames a workgroup 42 and 63. The compiled plan of 7680 against the run-time one: 37.2 / 41.5 and
+// 54.7 / 57.3 us back to back; run-time plans before and now: n_fft 5120 56 -> 36 and 72 -> 52, 6144 60 -> 38 and 77 -> 55.
 constexpr int kFrameTw = 2048;                         // full tables up to this n
 
 // Dynamic LDS: JOBS slots of frame_slot(M) float2, then the twiddles, then (iSTFT) the window.
