@@ -905,7 +905,8 @@ __global__ __launch_bounds__(kMixedThreads * FPB) void istft_frames_mixed_kernel
 // bytes of a row; JOBS = 16 frames make runs of 128. With TPF <= 64 a frame is one wave's, so its
 // passes need no barrier. The twiddles are the full table of W_n^m in LDS for n <= 2048. Bound by VALU
 // issue: n_fft 960, hop 480, a minute of stereo f-major 120 -> 24.9 us (2.55 TB/s of the signal and the
-// spectrum; 14.8 us of it VALU issue, 5.7 the CU's LDS), iSTFT 143 -> 32.2 (24.3 and 7.3); n_fft 320, hop 80, 12,502 frames 95 -> 15.3 and 109 -> 17.2.
+// spectrum; 14.8 us of it VALU issue, 5.7 the CU's LDS), iSTFT 143 -> 32.2 (24.3 and 7.3); n_fft 320, hop 80,
+// 12,502 frames 95 -> 15.3 and 109 -> 17.2.
 // With 128 and 256 threads a frame (n up to 7680 and 8192) the passes have barriers, and what counts is the one LDS
 // buffer a frame: two workgroups of 2 frames a CU, where stft_mixed_kernel's two ping-pong buffers held 2 frames in
 // all. n_fft 7680, 2,048 frames f-major: STFT 53 -> 39 us (23 of them VALU issue, 42 % of the wave time in waits),
@@ -1448,7 +1449,7 @@ template <int N, int JOBS>
 bool istft_runs_gain(const IstftArgs& t, long long tiles, long long runs) {
     if (t.layout == STX_SPEC_T_MAJOR || N < 1024 || N > 4096) return true;
     const long long span = t.tile_len % t.hop == 0 ? t.tile_len / t.hop + (N - 1) / t.hop : (t.tile_len + N - 2) / t.hop + 1;
-    const long long resident = istft_resident<N, JOBS>();
+    const long long resident = std::max(1LL, istft_resident<N, JOBS>());
     const long long rounds = (tiles + resident - 1) / resident * ((span + JOBS - 1) / JOBS);
     return runs * JOBS <= 2 * rounds * istft_run_jobs<N>();
 }
